@@ -72,7 +72,8 @@ void Precond<T>::factor(const std::vector<FactorJob>& jobs)
     const bool same = jobs.size() == jobs_host_.size() &&
                       std::equal(jobs.begin(), jobs.end(), jobs_host_.begin(), [](const FactorJob& a, const FactorJob& b) {
                           return a.start == b.start && a.len == b.len && a.dir == b.dir && a.boost == b.boost &&
-                                 a.boost_last == b.boost_last && a.buf == b.buf && a.kb == b.kb && a.boff == b.boff;
+                                 a.boost_last == b.boost_last && a.buf == b.buf && a.kb == b.kb && a.boff == b.boff &&
+                                 a.tab == b.tab;
                       });
     if (!same) {
         jobs_.resize(jobs.size());
@@ -85,6 +86,63 @@ void Precond<T>::factor(const std::vector<FactorJob>& jobs)
     for (const FactorJob& j : jobs) max_len = std::max(max_len, (int64_t)j.len);
     launch_band_factor<T>(B_.get(), Bul_.get(), sep_in_ ? Bin_.get() : nullptr, k, jobs_.get(), (int)jobs.size(),
                           max_len, stream);
+    make_tables(B_.get(), Bul_.get(), k, 0, (int)jobs.size(), max_len);
+}
+
+template <class T>
+void Precond<T>::begin_tables(int ranges, int kmax, bool with_ul)
+{
+    tabs_on_ = sweep_max_nbuf<T>(kmax) > 0;
+    if (!tabs_on_) {
+        tab_[0].release();
+        tab_[1].release();
+        return;
+    }
+    tab_stride_ = sweep_tab_elems<T>(n, ranges);
+    try {
+        tab_[0].resize((size_t)(2 * tab_stride_));
+        if (with_ul) tab_[1].resize((size_t)(2 * tab_stride_));
+        else tab_[1].release();
+    } catch (const Error& e) {
+        if (e.code != SAP_ERR_OOM) throw;
+        tab_[0].release();
+        tab_[1].release();
+        tabs_on_ = false;
+    }
+}
+
+template <class T>
+void Precond<T>::make_tables(const T* b0, const T* b1, int kl, size_t first, int njobs, int64_t max_len)
+{
+    if (!tabs_on_) return;
+    launch_sweep_tables<T>(b0, b1, kl, jobs_.get() + first, njobs, max_len, tab_[0].get(), tab_[1].get(), tab_stride_,
+                           stream);
+}
+
+template <class T>
+SweepTabs<T> Precond<T>::tabs() const
+{
+    SweepTabs<T> t;
+    if (!tabs_on_) return t;
+    t.lu1 = tab_[0].get();
+    t.lu2 = t.lu1 + tab_stride_;
+    if (tab_[1].get()) {
+        t.ul1 = tab_[1].get();
+        t.ul2 = t.ul1 + tab_stride_;
+    }
+    return t;
+}
+
+template <class T>
+SweepTabs<T> Precond<T>::range_tabs(int64_t start, int range) const
+{
+    SweepTabs<T> t = tabs();
+    if (!t.lu1) return t;
+    const int64_t off = sweep_tab_elems<T>(start, range);
+    t.lu1 += off;
+    t.lu2 += off;
+    t.ul1 = t.ul2 = nullptr;
+    return t;
 }
 
 template <class T>
@@ -659,7 +717,7 @@ void Precond<T>::var_spikes()
             pi.bounds(p, s, len);
             std::vector<SweepJob> one;
             size_t l = 0;
-            const int mode = sweep_range_job_append<T>(one, l, Bv_.get() + vboff_[p], vks_[p], 0, len,
+            const int mode = sweep_range_job_append<T>(one, l, Bv_.get() + vboff_[p], range_tabs(s, p), vks_[p], 0, len,
                                                        scr.get() + (int64_t)j * stride, len, 0, 0, 1);
             one[0].voff = one[0].ooff = (int64_t)j * stride;
             by_mode[mode].push_back(one[0]);
@@ -712,13 +770,14 @@ int Precond<T>::var_factor_steps()
     for (const auto& o : order) {
         int64_t s, len;
         pi.bounds(o.second, s, len);
-        FactorJob J{0, len, 1, 1, 1, 0, vks_[o.second], vboff_[o.second]};
+        FactorJob J{0, len, 1, 1, 1, 0, vks_[o.second], vboff_[o.second], sweep_tab_block<T>(s, o.second)};
         jobs.push_back(J);
     }
     const bool same = jobs.size() == jobs_host_.size() &&
                       std::equal(jobs.begin(), jobs.end(), jobs_host_.begin(), [](const FactorJob& a, const FactorJob& b) {
                           return a.start == b.start && a.len == b.len && a.dir == b.dir && a.boost == b.boost &&
-                                 a.boost_last == b.boost_last && a.buf == b.buf && a.kb == b.kb && a.boff == b.boff;
+                                 a.boost_last == b.boost_last && a.buf == b.buf && a.kb == b.kb && a.boff == b.boff &&
+                                 a.tab == b.tab;
                       });
     if (!same) {
         jobs_.resize(jobs.size());
@@ -726,6 +785,7 @@ int Precond<T>::var_factor_steps()
                                      stream));
         jobs_host_ = jobs;
     }
+    begin_tables(P, *std::max_element(vks_.begin(), vks_.end()), false);
     tm_.mark(3, stream);
     {
         ProfScope ps(prof, "band_factor");
@@ -740,6 +800,7 @@ int Precond<T>::var_factor_steps()
                 ++b;
             }
             launch_band_factor<T>(Bv_.get(), Bv_.get(), nullptr, kmax, jobs_.get() + a, (int)(b - a), max_len, stream);
+            make_tables(Bv_.get(), Bv_.get(), kmax, a, (int)(b - a), max_len);
             a = b;
         }
     }
@@ -804,8 +865,8 @@ typename Precond<T>::VJobs& Precond<T>::var_jobs(int nr, int64_t ldv, int64_t ld
         std::vector<SweepJob> one;
         size_t lds = 0;
         int mode = 0;
-        if (!sweep_jobs_append<T>(one, lds, Bp, Bp, vks_[p], PartInfo{len, 1}, 0, nullptr, scr + nr * s, s, ldv, s,
-                                  ldz, nr, 0, 0, &mode))
+        if (!sweep_jobs_append<T>(one, lds, Bp, range_tabs(s, p), vks_[p], PartInfo{len, 1}, scr + nr * s, s, ldv, s,
+                                  ldz, nr, 0, &mode))
             throw Error(SAP_ERR_HIP, "variable-bandwidth sweep job table");
         by_mode[mode].insert(by_mode[mode].end(), one.begin(), one.end());
         J.lds[mode] = std::max(J.lds[mode], lds);
@@ -925,19 +986,23 @@ int Precond<T>::bcr_factor_steps()
     bjobs_[0].nr = bjobs_[1].nr = 0;   // the sweep job tables are built again for these blocks
     const int boost = (k >= 70) || cfg.safeFactorization;
     const int boost_last = (k >= 70);
+    begin_tables((int)nblk, k, false);
+    auto bjob = [&](int b) -> FactorJob {
+        return {bblk_[b].start, bblk_[b].len, 1, boost, boost_last, 0, 0, 0, sweep_tab_block<T>(bblk_[b].start, b)};
+    };
     tm_.mark(3, stream);
     {
         ProfScope ps(prof, "band_factor");
         launch_bcr_extract<T>(B_.get(), k, bblk_d_.get(), (int)nblk, bCL_.get(), bCU_.get(), stream);
         for (const BcrLevel& L : blev_) {
             std::vector<FactorJob> jobs;
-            for (const BcrElim& E : L.el) jobs.push_back({bblk_[E.e].start, bblk_[E.e].len, 1, boost, boost_last, 0});
+            for (const BcrElim& E : L.el) jobs.push_back(bjob(E.e));
             factor(jobs);
             launch_bcr_level_setup<T>(B_.get(), k, bblk_d_.get(), L.d.get(), (int)L.el.size(), max_len, bCL_.get(),
                                       bCU_.get(), bUA_.get(), bLC_.get(), stream);
         }
         std::vector<FactorJob> jobs;
-        for (int b : bfinal_) jobs.push_back({bblk_[b].start, bblk_[b].len, 1, boost, boost_last, 0});
+        for (int b : bfinal_) jobs.push_back(bjob(b));
         factor(jobs);
     }
     tm_.mark(4, stream);
@@ -963,7 +1028,8 @@ typename Precond<T>::BcrJobs& Precond<T>::bcr_jobs(int nr, T* scr)
     J.start.clear();
     J.count.clear();
     auto add = [&](int b) {
-        mode = sweep_range_job_append<T>(jobs, lds, B_.get(), k, bblk_[b].start, bblk_[b].len, scr, n, n, n, nr);
+        mode = sweep_range_job_append<T>(jobs, lds, B_.get(), range_tabs(bblk_[b].start, b), k, bblk_[b].start,
+                                         bblk_[b].len, scr, n, n, n, nr);
     };
     for (const BcrLevel& L : blev_) {
         J.start.push_back(jobs.size());
@@ -1047,13 +1113,14 @@ int Precond<T>::factor_band_steps()
     // no stored pivot can be below 1e-7, so the check is skipped.
     const bool check_pivots = !cfg.safeFactorization && !(boost && boost_last);
 
+    begin_tables(P, k, lu_ul() && spike_active());
     const size_t kk = (size_t)k * k;
     if (!spike_active()) {
         std::vector<FactorJob> jobs;
         for (int p = 0; p < P; ++p) {
             int64_t s, len;
             pi.bounds(p, s, len);
-            jobs.push_back({s, len, 1, boost, boost_last, 0});
+            jobs.push_back({s, len, 1, boost, boost_last, 0, 0, 0, sweep_tab_block<T>(s, p)});
         }
         tm_.mark(3, stream);
         factor(jobs);
@@ -1100,12 +1167,12 @@ int Precond<T>::factor_band_steps()
         for (int p = 0; p < P - 1; ++p) {
             int64_t s, len;
             pi.bounds(p, s, len);
-            jobs.push_back({s, len, 1, boost, boost_last, 0});
+            jobs.push_back({s, len, 1, boost, boost_last, 0, 0, 0, sweep_tab_block<T>(s, p)});
         }
         for (int p = 1; p < P; ++p) {
             int64_t s, len;
             pi.bounds(p, s, len);
-            jobs.push_back({s, len, -1, boost, boost_last, 1});
+            jobs.push_back({s, len, -1, boost, boost_last, 1, 0, 0, sweep_tab_block<T>(s, p)});
         }
         // With every pivot boosted (no factorization can fail), also the LU
         // of the last partition and the UL of the first (two more jobs
@@ -1116,8 +1183,8 @@ int Precond<T>::factor_band_steps()
         if (split_) {
             int64_t s0, l0;
             pi.bounds(0, s0, l0);
-            jobs.push_back({s_last, l_last, 1, boost, boost_last, 0});
-            jobs.push_back({s0, l0, -1, boost, boost_last, 1});
+            jobs.push_back({s_last, l_last, 1, boost, boost_last, 0, 0, 0, sweep_tab_block<T>(s_last, P - 1)});
+            jobs.push_back({s0, l0, -1, boost, boost_last, 1, 0, 0, sweep_tab_block<T>(s0, 0)});
         }
         scr1_.resize(n);
     } else {
@@ -1126,7 +1193,7 @@ int Precond<T>::factor_band_steps()
         for (int p = 0; p < P; ++p) {
             int64_t s, len;
             pi.bounds(p, s, len);
-            jobs.push_back({s, len, 1, boost, boost_last, 0});
+            jobs.push_back({s, len, 1, boost, boost_last, 0, 0, 0, sweep_tab_block<T>(s, p)});
         }
     }
     factor(jobs);
@@ -1220,10 +1287,10 @@ void Precond<T>::solve_band(const double* v, double* z)
     if (spike_active()) {
         if (lu_ul()) {
             ProfScope ps(prof, "sweep_interface");
-            launch_sweep_interface<T>(B_.get(), Bul_.get(), k, pi, v, g_.get(), scr0_.get(), scr1_.get(), stream, rh);
+            launch_sweep_interface<T>(B_.get(), Bul_.get(), tabs(), k, pi, v, g_.get(), scr0_.get(), scr1_.get(), stream, rh);
         } else {
             ProfScope ps(prof, "sweep_interface");
-            launch_sweep_full<T>(B_.get(), B_.get(), k, pi, 0, v, nullptr, nullptr, g_.get(), scr0_.get(), stream, rh);
+            launch_sweep_full<T>(B_.get(), B_.get(), tabs(), k, pi, 0, v, nullptr, nullptr, g_.get(), scr0_.get(), stream, rh);
         }
         wait_spikes();
         {
@@ -1234,11 +1301,11 @@ void Precond<T>::solve_band(const double* v, double* z)
         ProfScope ps(prof, "sweep_full");
         Rhs r2 = rh;
         if (split_ && lu_ul()) r2.split_scr = scr1_.get();
-        launch_sweep_full<T>(B_.get(), Bul_.get(), k, pi, lu_ul() ? 1 : 0, v, corr_.get(), z, nullptr, scr0_.get(),
+        launch_sweep_full<T>(B_.get(), Bul_.get(), tabs(), k, pi, lu_ul() ? 1 : 0, v, corr_.get(), z, nullptr, scr0_.get(),
                              stream, r2);
     } else {
         ProfScope ps(prof, "sweep_full");
-        launch_sweep_full<T>(B_.get(), B_.get(), k, pi, 0, v, nullptr, z, nullptr, scr0_.get(), stream, rh);
+        launch_sweep_full<T>(B_.get(), B_.get(), tabs(), k, pi, 0, v, nullptr, z, nullptr, scr0_.get(), stream, rh);
     }
 }
 
@@ -1284,8 +1351,8 @@ bool Precond<T>::append_sweep_jobs(std::vector<SweepJob>& jobs, size_t& lds, int
 {
     if (cfg.precondType == SAP_None || reorder_ || spike_active() || k == 0 || bcr_) return false;
     reserve_multi(nr);
-    return sweep_jobs_append<T>(jobs, lds, B_.get(), B_.get(), k, PartInfo{n, P}, 0, nullptr, scr0m_.get(), voff, n,
-                                ooff, n, nr, gate0, nbuf_);
+    return sweep_jobs_append<T>(jobs, lds, B_.get(), tabs(), k, PartInfo{n, P}, scr0m_.get(), voff, n, ooff, n, nr,
+                                gate0);
 }
 
 template <class T>
@@ -1337,10 +1404,10 @@ void Precond<T>::solve_band_multi(const double* V, int64_t ldv, double* Z, int64
     if (spike_active()) {
         if (lu_ul()) {
             ProfScope ps(prof, "sweep_interface");
-            launch_sweep_interface<T>(B_.get(), Bul_.get(), k, pi, V, gm_.get(), scr0m_.get(), scr1m_.get(), stream, rh);
+            launch_sweep_interface<T>(B_.get(), Bul_.get(), tabs(), k, pi, V, gm_.get(), scr0m_.get(), scr1m_.get(), stream, rh);
         } else {
             ProfScope ps(prof, "sweep_interface");
-            launch_sweep_full<T>(B_.get(), B_.get(), k, pi, 0, V, nullptr, nullptr, gm_.get(), scr0m_.get(), stream, rh);
+            launch_sweep_full<T>(B_.get(), B_.get(), tabs(), k, pi, 0, V, nullptr, nullptr, gm_.get(), scr0m_.get(), stream, rh);
         }
         wait_spikes();
         {
@@ -1351,11 +1418,11 @@ void Precond<T>::solve_band_multi(const double* V, int64_t ldv, double* Z, int64
         ProfScope ps(prof, "sweep_full");
         Rhs r2 = rh;
         if (split_ && lu_ul()) r2.split_scr = scr1m_.get();
-        launch_sweep_full<T>(B_.get(), Bul_.get(), k, pi, lu_ul() ? 1 : 0, V, corrm_.get(), Z, nullptr, scr0m_.get(),
+        launch_sweep_full<T>(B_.get(), Bul_.get(), tabs(), k, pi, lu_ul() ? 1 : 0, V, corrm_.get(), Z, nullptr, scr0m_.get(),
                              stream, r2);
     } else {
         ProfScope ps(prof, "sweep_full");
-        launch_sweep_full<T>(B_.get(), B_.get(), k, pi, 0, V, nullptr, Z, nullptr, scr0m_.get(), stream, rh);
+        launch_sweep_full<T>(B_.get(), B_.get(), tabs(), k, pi, 0, V, nullptr, Z, nullptr, scr0m_.get(), stream, rh);
     }
 }
 

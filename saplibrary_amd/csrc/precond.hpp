@@ -200,6 +200,18 @@ public:
 
 private:
     DevBuf<T> B_, Bul_, offB_, offC_, WV_, S_, Sinv_, g_, corr_, scr0_, scr1_;
+    // the staged sweeps' tables (the LU and the UL band's, stage 1 then
+    // stage 2); without memory for them (tabs_on_ false) the
+    // sweeps are the plain blocked ones
+    DevBuf<T> tab_[2];
+    int64_t tab_stride_ = 0;
+    bool tabs_on_ = false;
+    // sizes the tables for `ranges` factored ranges over the n rows
+    void begin_tables(int ranges, int kmax, bool with_ul);
+    void make_tables(const T* b0, const T* b1, int kl, size_t first, int njobs, int64_t max_len);
+    // the tables of range `range` starting at row `start` (LU band)
+    SweepTabs<T> range_tabs(int64_t start, int range) const;
+    SweepTabs<T> tabs() const;
     DevBuf<FactorJob> jobs_;
     std::vector<FactorJob> jobs_host_;   // what jobs_ holds
     DevBuf<int> flag_;

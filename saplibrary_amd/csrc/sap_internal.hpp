@@ -232,6 +232,7 @@ struct FactorJob {          // one banded LU (dir = +1) or UL (dir = -1) of a pa
     int     kb;             // the job's half-bandwidth (0: the launch's k)
     int64_t boff;           // element offset of the job's band in its buffer
                             // (a partition stored in a band of its own width)
+    int64_t tab;            // first block of the job's sweep tables (sweep_tab_block)
 };
 // max_len: longest partition among the jobs.  Bin: the unfactored band the
 // jobs read (the factors go to B0 / B1), or null for in-place factorization;
@@ -318,6 +319,25 @@ struct Rhs {
     // stage-1 values go to this second scratch (same layout as scr)
     void* split_scr = nullptr;
 };
+// Tables of the factors' diagonal blocks (inverted), sub-diagonal blocks and
+// pivots, which the staged sweeps multiply with: of the LU factors for the sweep in the direction of the
+// factorization (1) and against it (2), and of the UL factors the same.
+// Null pointers: the plain blocked sweeps, which substitute.
+template <class T>
+struct SweepTabs {
+    const T *lu1 = nullptr, *lu2 = nullptr, *ul1 = nullptr, *ul2 = nullptr;
+};
+// elements of one table over n rows cut into `ranges` consecutive ranges,
+// and the first block of the range that starts at row `start`
+template <class T>
+int64_t sweep_tab_elems(int64_t n, int ranges);
+template <class T>
+int64_t sweep_tab_block(int64_t start, int range);
+// Tables of the factored jobs: stage 1 at tab0 (buf 0) / tab1 (buf 1), stage
+// 2 stage_stride elements on.
+template <class T>
+void launch_sweep_tables(const T* B0, const T* B1, int k, const FactorJob* d_jobs, int njobs, int64_t max_len, T* tab0,
+                         T* tab1, int64_t stage_stride, hipStream_t st);
 // the staged sweeps' largest LDS block-buffer count for k (0: not staged)
 template <class T>
 int sweep_max_nbuf(int k);
@@ -328,6 +348,7 @@ int sweep_max_nbuf(int k);
 struct SweepJob {
     const void* B;        // the system's factor band (null: a padding job)
     const void* Bul;      // its UL band (last partition under LU_UL)
+    const void *t1, *t2;  // its sweep tables (SweepTabs)
     const void* corr;     // reduced-system corrections of this column, or null
     void* scr;            // n-element work vector of this column
     int64_t voff, ooff;
@@ -337,33 +358,34 @@ struct SweepJob {
 };
 // Appends nr jobs (column r: input V + r*ldv, output Z + r*ldo, scratch
 // scr + r*n, gate r) sweeping band rows [s0, s0 + len0) of B (half-bandwidth
-// k, n rows) as one system; returns the sweep variant (jobs of one launch
+// k, n rows; tabs: the range's own tables) as one system; returns the sweep variant (jobs of one launch
 // share it) and raises lds to what it needs.
 template <class T>
-int sweep_range_job_append(std::vector<SweepJob>& jobs, size_t& lds, const T* B, int k, int64_t s0, int64_t len0,
-                           T* scr, int64_t n, int64_t ldv, int64_t ldo, int nr);
+int sweep_range_job_append(std::vector<SweepJob>& jobs, size_t& lds, const T* B, const SweepTabs<T>& tabs, int k,
+                           int64_t s0, int64_t len0, T* scr, int64_t n, int64_t ldv, int64_t ldo, int nr);
 // Appends the jobs of one system (nr columns at voff + r*ldv / ooff +
-// r*ldo, scr and corr holding nr consecutive blocks, gates gate0 + r) and
+// r*ldo, scr holding nr consecutive blocks, gates gate0 + r) and
 // raises lds to what they need.  Without mode_out: false when its width
 // does not take the staged sweep (nothing appended); with mode_out: any
 // width, *mode_out the sweep variant its jobs need (jobs of one launch
 // share it).  False for k = 0.
 template <class T>
-bool sweep_jobs_append(std::vector<SweepJob>& jobs, size_t& lds, const T* B, const T* Bul, int k, PartInfo pi,
-                       int last_is_ul, const T* corr, T* scr, int64_t voff, int64_t ldv, int64_t ooff, int64_t ldo,
-                       int nr, int gate0, int nbuf_req, int* mode_out = nullptr);
+bool sweep_jobs_append(std::vector<SweepJob>& jobs, size_t& lds, const T* B, const SweepTabs<T>& tabs, int k,
+                       PartInfo pi, T* scr, int64_t voff, int64_t ldv, int64_t ooff, int64_t ldo, int nr, int gate0,
+                       int* mode_out = nullptr);
 template <class T>
 void launch_sweep_full_jobs(const SweepJob* d_jobs, int njobs, size_t lds, const double* V, double* Z,
                             const int* gate, hipStream_t st, int mode = 2);
 template <class T>
-void launch_sweep_interface(const T* B, const T* Bul, int k, PartInfo pi, const double* v, T* g, T* scr0, T* scr1,
-                            hipStream_t st, const Rhs& rh = Rhs());
+void launch_sweep_interface(const T* B, const T* Bul, const SweepTabs<T>& tabs, int k, PartInfo pi, const double* v,
+                            T* g, T* scr0, T* scr1, hipStream_t st, const Rhs& rh = Rhs());
 template <class T>
 void launch_interface_solve(const T* WV, const T* Sinv, const T* offB, const T* offC, int k, PartInfo pi,
                             const T* g, T* corr, hipStream_t st, const Rhs& rh = Rhs());
 template <class T>
-void launch_sweep_full(const T* B, const T* Bul, int k, PartInfo pi, int last_is_ul, const double* v, const T* corr,
-                       double* outd, T* outt, T* scr, hipStream_t st, const Rhs& rh = Rhs());
+void launch_sweep_full(const T* B, const T* Bul, const SweepTabs<T>& tabs, int k, PartInfo pi, int last_is_ul,
+                       const double* v, const T* corr, double* outd, T* outt, T* scr, hipStream_t st,
+                       const Rhs& rh = Rhs());
 template <class T>
 void launch_diag_divide(const T* B, int64_t n, const double* v, double* out, hipStream_t st, const Rhs& rh = Rhs());
 // zeros in A[0, na) and B[0, nb) (B may be null when nb = 0)
