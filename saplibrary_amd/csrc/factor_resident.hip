@@ -8,6 +8,7 @@
 #include "sap_internal.hpp"
 
 #include <climits>
+#include <type_traits>
 
 namespace sap_amd {
 
@@ -25,38 +26,346 @@ namespace {
 // columns and U rows, and the slots they free take the tiles that enter, so
 // every band entry is read from HBM once and every factor entry written once.
 // Per panel:
-//   A0. the slots of the 32 x 32 diagonal block are copied to LDS;
-//   B1. wavefront 0 factors that block in registers, one row per lane, pivot
-//       rows broadcast with readlane, boosting at pivot time, while
-//   A.  the other wavefronts (and wavefront 0 after B1) copy the other panel
-//       column and U row slots to LDS, start loading the entering tiles
-//       (first used one panel later) and store the previous panel's factors
-//       from the other LDS buffer;
-//   B2. 16(KT-2) threads solve L21 = A21 U11^-1 row by row, another 16(KT-2)
-//       threads U12 = L11^-1 A12 column by column (unit L11);
+//   A.  the slots of the panel's columns and U rows are copied to LDS, and
+//       start loading the entering tiles (first used one panel later);
+//   B.  the panel is factored in two sub-panels of 16 columns.  The first
+//       wavefronts hold the rows below the sub-panel's diagonal block, one
+//       per lane (L), as many others the columns right of it (U), and every
+//       16-lane row of every wavefront holds a copy of the diagonal block
+//       itself, one row per lane: each factors its copy (boosting at pivot
+//       time) and applies every elimination step to its own row or column at
+//       once, with the pivot row (the multipliers) broadcast from the copy
+//       inside the lane row by DPP.  So the diagonal block's LU and both
+//       triangular solves are one pass of 16 steps, with no exchange between
+//       wavefronts.  Between the sub-panels the first one's contribution to
+//       the second's columns and rows goes through the matrix cores;
 //   C.  trailing tiles += (-L21) U12 on the matrix cores
 //       (v_mfma_f32_16x16x4f32 / v_mfma_f64_16x16x4f64, the 32 panel columns
-//       split over the four lane groups).  Tiles are kept transposed in the
-//       accumulators (the update is acc^T += U12^T (-L21)^T), which makes each
-//       tile load read whole 16-row column segments.
+//       split over the four lane groups), and the panel's factors go out;
+//       wavefronts w and w + 4 share a SIMD, and one does its stores while
+//       the other multiplies.  Tiles are kept transposed in the accumulators
+//       (the update is acc^T += U12^T (-L21)^T), which makes each tile load
+//       read whole 16-row column segments.
 // Outside the band every stored value is an exact zero, so the padded tiles
 // never create fill-in.  The wavefronts exchange data only through LDS (each
 // tile load is consumed by the wavefront that issued it; factor stores are
-// not read back), so the barriers do not wait for global memory, and all
-// global accesses of a panel are issued in phase A, where they have B1 and
-// B2 to complete.  Factors are stored as L (unit), D, U' like the other
-// factorization kernels; the multipliers use the pivot's reciprocal.
+// not read back), so the barriers do not wait for global memory.  Factors are
+// stored as L (unit), D, U' like the other factorization kernels; the
+// multipliers use the pivot's reciprocal.
+// What bounds it: two wavefronts on a SIMD, each running a chain of dependent
+// instructions (8 cycles apiece, 12 while the other one multiplies), so time
+// goes with the instructions per panel, not with bytes (k = 200: 0.6 TB/s) and
+// only for the widest windows with the matrix cores (k = 200: 9.2k of 40k
+// cycles a panel).  Both triangular solves in one pass over register-held rows
+// and columns, instead of a diagonal LU by one wavefront followed by solves
+// out of LDS, took the factorizations of both directions from 3.15 to 2.58 ms
+// (n = 200000, k = 50, 16 partitions, FP32), 8.53 to 8.28 ms (n = 1000000,
+// k = 200, 64 partitions), and in FP64 (n = 100000, 8 partitions) from 5.80
+// to 2.75 ms at k = 16 and 8.65 to 5.54 ms at k = 100.
 // ---------------------------------------------------------------------------
-__device__ inline float lane_bcast(float v, int src)
+// acc -= (lane N of the 16-lane row of src) * m.  hipcc does not fold the
+// broadcast into the multiply-add, so it is written out; an instruction that
+// broadcasts must not follow the one that wrote its source by less than two
+// wait states, hence the s_nop that begins every group.
+// a[i] -= (lane N of the row of c[i]) * m; in place (c = a); a[i] -= (lane
+// N + i of the row of c) * m, for groups of 8, 4, 2 and 1
+template <int N>
+__device__ __forceinline__ void bc_rows8(float* a, const float* c, float m)
 {
-    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), src));
+    asm volatile("s_nop 1\n\t"
+                 "v_fmac_f32_dpp %0, -%8, %16 row_newbcast:%17 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f32_dpp %1, -%9, %16 row_newbcast:%17 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f32_dpp %2, -%10, %16 row_newbcast:%17 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f32_dpp %3, -%11, %16 row_newbcast:%17 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f32_dpp %4, -%12, %16 row_newbcast:%17 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f32_dpp %5, -%13, %16 row_newbcast:%17 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f32_dpp %6, -%14, %16 row_newbcast:%17 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f32_dpp %7, -%15, %16 row_newbcast:%17 row_mask:0xf bank_mask:0xf"
+                 : "+&v"(a[0]), "+&v"(a[1]), "+&v"(a[2]), "+&v"(a[3]), "+&v"(a[4]), "+&v"(a[5]), "+&v"(a[6]), "+&v"(a[7])
+                 : "v"(c[0]), "v"(c[1]), "v"(c[2]), "v"(c[3]), "v"(c[4]), "v"(c[5]), "v"(c[6]), "v"(c[7]), "v"(m), "n"(N));
+}
+template <int N>
+__device__ __forceinline__ void bc_rows8(double* a, const double* c, double m)
+{
+    asm volatile("s_nop 1\n\t"
+                 "v_fmac_f64_dpp %0, -%8, %16 row_newbcast:%17 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f64_dpp %1, -%9, %16 row_newbcast:%17 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f64_dpp %2, -%10, %16 row_newbcast:%17 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f64_dpp %3, -%11, %16 row_newbcast:%17 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f64_dpp %4, -%12, %16 row_newbcast:%17 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f64_dpp %5, -%13, %16 row_newbcast:%17 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f64_dpp %6, -%14, %16 row_newbcast:%17 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f64_dpp %7, -%15, %16 row_newbcast:%17 row_mask:0xf bank_mask:0xf"
+                 : "+&v"(a[0]), "+&v"(a[1]), "+&v"(a[2]), "+&v"(a[3]), "+&v"(a[4]), "+&v"(a[5]), "+&v"(a[6]), "+&v"(a[7])
+                 : "v"(c[0]), "v"(c[1]), "v"(c[2]), "v"(c[3]), "v"(c[4]), "v"(c[5]), "v"(c[6]), "v"(c[7]), "v"(m), "n"(N));
+}
+template <int N>
+__device__ __forceinline__ void bc_rows4(float* a, const float* c, float m)
+{
+    asm volatile("s_nop 1\n\t"
+                 "v_fmac_f32_dpp %0, -%4, %8 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f32_dpp %1, -%5, %8 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f32_dpp %2, -%6, %8 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f32_dpp %3, -%7, %8 row_newbcast:%9 row_mask:0xf bank_mask:0xf"
+                 : "+&v"(a[0]), "+&v"(a[1]), "+&v"(a[2]), "+&v"(a[3])
+                 : "v"(c[0]), "v"(c[1]), "v"(c[2]), "v"(c[3]), "v"(m), "n"(N));
+}
+template <int N>
+__device__ __forceinline__ void bc_rows4(double* a, const double* c, double m)
+{
+    asm volatile("s_nop 1\n\t"
+                 "v_fmac_f64_dpp %0, -%4, %8 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f64_dpp %1, -%5, %8 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f64_dpp %2, -%6, %8 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f64_dpp %3, -%7, %8 row_newbcast:%9 row_mask:0xf bank_mask:0xf"
+                 : "+&v"(a[0]), "+&v"(a[1]), "+&v"(a[2]), "+&v"(a[3])
+                 : "v"(c[0]), "v"(c[1]), "v"(c[2]), "v"(c[3]), "v"(m), "n"(N));
+}
+template <int N>
+__device__ __forceinline__ void bc_rows2(float* a, const float* c, float m)
+{
+    asm volatile("s_nop 1\n\t"
+                 "v_fmac_f32_dpp %0, -%2, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f32_dpp %1, -%3, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf"
+                 : "+&v"(a[0]), "+&v"(a[1])
+                 : "v"(c[0]), "v"(c[1]), "v"(m), "n"(N));
+}
+template <int N>
+__device__ __forceinline__ void bc_rows2(double* a, const double* c, double m)
+{
+    asm volatile("s_nop 1\n\t"
+                 "v_fmac_f64_dpp %0, -%2, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f64_dpp %1, -%3, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf"
+                 : "+&v"(a[0]), "+&v"(a[1])
+                 : "v"(c[0]), "v"(c[1]), "v"(m), "n"(N));
+}
+template <int N>
+__device__ __forceinline__ void bc_rows1(float* a, const float* c, float m)
+{
+    asm volatile("s_nop 1\n\t"
+                 "v_fmac_f32_dpp %0, -%1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf"
+                 : "+&v"(a[0])
+                 : "v"(c[0]), "v"(m), "n"(N));
+}
+template <int N>
+__device__ __forceinline__ void bc_rows1(double* a, const double* c, double m)
+{
+    asm volatile("s_nop 1\n\t"
+                 "v_fmac_f64_dpp %0, -%1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf"
+                 : "+&v"(a[0])
+                 : "v"(c[0]), "v"(m), "n"(N));
+}
+template <int N>
+__device__ __forceinline__ void bc_self8(float* a, float m)
+{
+    asm volatile("s_nop 1\n\t"
+                 "v_fmac_f32_dpp %0, -%0, %8 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f32_dpp %1, -%1, %8 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f32_dpp %2, -%2, %8 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f32_dpp %3, -%3, %8 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f32_dpp %4, -%4, %8 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f32_dpp %5, -%5, %8 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f32_dpp %6, -%6, %8 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f32_dpp %7, -%7, %8 row_newbcast:%9 row_mask:0xf bank_mask:0xf"
+                 : "+&v"(a[0]), "+&v"(a[1]), "+&v"(a[2]), "+&v"(a[3]), "+&v"(a[4]), "+&v"(a[5]), "+&v"(a[6]), "+&v"(a[7])
+                 : "v"(m), "n"(N));
+}
+template <int N>
+__device__ __forceinline__ void bc_self8(double* a, double m)
+{
+    asm volatile("s_nop 1\n\t"
+                 "v_fmac_f64_dpp %0, -%0, %8 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f64_dpp %1, -%1, %8 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f64_dpp %2, -%2, %8 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f64_dpp %3, -%3, %8 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f64_dpp %4, -%4, %8 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f64_dpp %5, -%5, %8 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f64_dpp %6, -%6, %8 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f64_dpp %7, -%7, %8 row_newbcast:%9 row_mask:0xf bank_mask:0xf"
+                 : "+&v"(a[0]), "+&v"(a[1]), "+&v"(a[2]), "+&v"(a[3]), "+&v"(a[4]), "+&v"(a[5]), "+&v"(a[6]), "+&v"(a[7])
+                 : "v"(m), "n"(N));
+}
+template <int N>
+__device__ __forceinline__ void bc_self4(float* a, float m)
+{
+    asm volatile("s_nop 1\n\t"
+                 "v_fmac_f32_dpp %0, -%0, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f32_dpp %1, -%1, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f32_dpp %2, -%2, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f32_dpp %3, -%3, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf"
+                 : "+&v"(a[0]), "+&v"(a[1]), "+&v"(a[2]), "+&v"(a[3])
+                 : "v"(m), "n"(N));
+}
+template <int N>
+__device__ __forceinline__ void bc_self4(double* a, double m)
+{
+    asm volatile("s_nop 1\n\t"
+                 "v_fmac_f64_dpp %0, -%0, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f64_dpp %1, -%1, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f64_dpp %2, -%2, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f64_dpp %3, -%3, %4 row_newbcast:%5 row_mask:0xf bank_mask:0xf"
+                 : "+&v"(a[0]), "+&v"(a[1]), "+&v"(a[2]), "+&v"(a[3])
+                 : "v"(m), "n"(N));
+}
+template <int N>
+__device__ __forceinline__ void bc_self2(float* a, float m)
+{
+    asm volatile("s_nop 1\n\t"
+                 "v_fmac_f32_dpp %0, -%0, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f32_dpp %1, -%1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf"
+                 : "+&v"(a[0]), "+&v"(a[1])
+                 : "v"(m), "n"(N));
+}
+template <int N>
+__device__ __forceinline__ void bc_self2(double* a, double m)
+{
+    asm volatile("s_nop 1\n\t"
+                 "v_fmac_f64_dpp %0, -%0, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f64_dpp %1, -%1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf"
+                 : "+&v"(a[0]), "+&v"(a[1])
+                 : "v"(m), "n"(N));
+}
+template <int N>
+__device__ __forceinline__ void bc_self1(float* a, float m)
+{
+    asm volatile("s_nop 1\n\t"
+                 "v_fmac_f32_dpp %0, -%0, %1 row_newbcast:%2 row_mask:0xf bank_mask:0xf"
+                 : "+&v"(a[0])
+                 : "v"(m), "n"(N));
+}
+template <int N>
+__device__ __forceinline__ void bc_self1(double* a, double m)
+{
+    asm volatile("s_nop 1\n\t"
+                 "v_fmac_f64_dpp %0, -%0, %1 row_newbcast:%2 row_mask:0xf bank_mask:0xf"
+                 : "+&v"(a[0])
+                 : "v"(m), "n"(N));
+}
+template <int N>
+__device__ __forceinline__ void bc_cols8(float* a, float c, float m)
+{
+    asm volatile("s_nop 1\n\t"
+                 "v_fmac_f32_dpp %0, -%8, %9 row_newbcast:%10 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f32_dpp %1, -%8, %9 row_newbcast:%11 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f32_dpp %2, -%8, %9 row_newbcast:%12 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f32_dpp %3, -%8, %9 row_newbcast:%13 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f32_dpp %4, -%8, %9 row_newbcast:%14 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f32_dpp %5, -%8, %9 row_newbcast:%15 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f32_dpp %6, -%8, %9 row_newbcast:%16 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f32_dpp %7, -%8, %9 row_newbcast:%17 row_mask:0xf bank_mask:0xf"
+                 : "+&v"(a[0]), "+&v"(a[1]), "+&v"(a[2]), "+&v"(a[3]), "+&v"(a[4]), "+&v"(a[5]), "+&v"(a[6]), "+&v"(a[7])
+                 : "v"(c), "v"(m), "n"(N + 0), "n"(N + 1), "n"(N + 2), "n"(N + 3), "n"(N + 4), "n"(N + 5), "n"(N + 6), "n"(N + 7));
+}
+template <int N>
+__device__ __forceinline__ void bc_cols8(double* a, double c, double m)
+{
+    asm volatile("s_nop 1\n\t"
+                 "v_fmac_f64_dpp %0, -%8, %9 row_newbcast:%10 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f64_dpp %1, -%8, %9 row_newbcast:%11 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f64_dpp %2, -%8, %9 row_newbcast:%12 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f64_dpp %3, -%8, %9 row_newbcast:%13 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f64_dpp %4, -%8, %9 row_newbcast:%14 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f64_dpp %5, -%8, %9 row_newbcast:%15 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f64_dpp %6, -%8, %9 row_newbcast:%16 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f64_dpp %7, -%8, %9 row_newbcast:%17 row_mask:0xf bank_mask:0xf"
+                 : "+&v"(a[0]), "+&v"(a[1]), "+&v"(a[2]), "+&v"(a[3]), "+&v"(a[4]), "+&v"(a[5]), "+&v"(a[6]), "+&v"(a[7])
+                 : "v"(c), "v"(m), "n"(N + 0), "n"(N + 1), "n"(N + 2), "n"(N + 3), "n"(N + 4), "n"(N + 5), "n"(N + 6), "n"(N + 7));
+}
+template <int N>
+__device__ __forceinline__ void bc_cols4(float* a, float c, float m)
+{
+    asm volatile("s_nop 1\n\t"
+                 "v_fmac_f32_dpp %0, -%4, %5 row_newbcast:%6 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f32_dpp %1, -%4, %5 row_newbcast:%7 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f32_dpp %2, -%4, %5 row_newbcast:%8 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f32_dpp %3, -%4, %5 row_newbcast:%9 row_mask:0xf bank_mask:0xf"
+                 : "+&v"(a[0]), "+&v"(a[1]), "+&v"(a[2]), "+&v"(a[3])
+                 : "v"(c), "v"(m), "n"(N + 0), "n"(N + 1), "n"(N + 2), "n"(N + 3));
+}
+template <int N>
+__device__ __forceinline__ void bc_cols4(double* a, double c, double m)
+{
+    asm volatile("s_nop 1\n\t"
+                 "v_fmac_f64_dpp %0, -%4, %5 row_newbcast:%6 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f64_dpp %1, -%4, %5 row_newbcast:%7 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f64_dpp %2, -%4, %5 row_newbcast:%8 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f64_dpp %3, -%4, %5 row_newbcast:%9 row_mask:0xf bank_mask:0xf"
+                 : "+&v"(a[0]), "+&v"(a[1]), "+&v"(a[2]), "+&v"(a[3])
+                 : "v"(c), "v"(m), "n"(N + 0), "n"(N + 1), "n"(N + 2), "n"(N + 3));
+}
+template <int N>
+__device__ __forceinline__ void bc_cols2(float* a, float c, float m)
+{
+    asm volatile("s_nop 1\n\t"
+                 "v_fmac_f32_dpp %0, -%2, %3 row_newbcast:%4 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f32_dpp %1, -%2, %3 row_newbcast:%5 row_mask:0xf bank_mask:0xf"
+                 : "+&v"(a[0]), "+&v"(a[1])
+                 : "v"(c), "v"(m), "n"(N + 0), "n"(N + 1));
+}
+template <int N>
+__device__ __forceinline__ void bc_cols2(double* a, double c, double m)
+{
+    asm volatile("s_nop 1\n\t"
+                 "v_fmac_f64_dpp %0, -%2, %3 row_newbcast:%4 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f64_dpp %1, -%2, %3 row_newbcast:%5 row_mask:0xf bank_mask:0xf"
+                 : "+&v"(a[0]), "+&v"(a[1])
+                 : "v"(c), "v"(m), "n"(N + 0), "n"(N + 1));
+}
+template <int N>
+__device__ __forceinline__ void bc_cols1(float* a, float c, float m)
+{
+    asm volatile("s_nop 1\n\t"
+                 "v_fmac_f32_dpp %0, -%1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf"
+                 : "+&v"(a[0])
+                 : "v"(c), "v"(m), "n"(N + 0));
+}
+template <int N>
+__device__ __forceinline__ void bc_cols1(double* a, double c, double m)
+{
+    asm volatile("s_nop 1\n\t"
+                 "v_fmac_f64_dpp %0, -%1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf"
+                 : "+&v"(a[0])
+                 : "v"(c), "v"(m), "n"(N + 0));
 }
 
-__device__ inline double lane_bcast(double v, int src)
+// the same for i = J .. 15
+template <int N, int J, class T>
+__device__ __forceinline__ void bc_rows(T (&a)[16], const T (&c)[16], T m)
+{
+    if constexpr (J + 7 < 16) { bc_rows8<N>(a + J, c + J, m); bc_rows<N, J + 8, T>(a, c, m); }
+    else if constexpr (J + 3 < 16) { bc_rows4<N>(a + J, c + J, m); bc_rows<N, J + 4, T>(a, c, m); }
+    else if constexpr (J + 1 < 16) { bc_rows2<N>(a + J, c + J, m); bc_rows<N, J + 2, T>(a, c, m); }
+    else if constexpr (J < 16) { bc_rows1<N>(a + J, c + J, m); }
+}
+template <int N, int J, class T>
+__device__ __forceinline__ void bc_self(T (&a)[16], T m)
+{
+    if constexpr (J + 7 < 16) { bc_self8<N>(a + J, m); bc_self<N, J + 8, T>(a, m); }
+    else if constexpr (J + 3 < 16) { bc_self4<N>(a + J, m); bc_self<N, J + 4, T>(a, m); }
+    else if constexpr (J + 1 < 16) { bc_self2<N>(a + J, m); bc_self<N, J + 2, T>(a, m); }
+    else if constexpr (J < 16) { bc_self1<N>(a + J, m); }
+}
+// u[i] -= (lane i of the row of c) * m for i = I .. 15
+template <int I, class T>
+__device__ __forceinline__ void bc_cols(T (&u)[16], T c, T m)
+{
+    if constexpr (I + 7 < 16) { bc_cols8<I>(u + I, c, m); bc_cols<I + 8, T>(u, c, m); }
+    else if constexpr (I + 3 < 16) { bc_cols4<I>(u + I, c, m); bc_cols<I + 4, T>(u, c, m); }
+    else if constexpr (I + 1 < 16) { bc_cols2<I>(u + I, c, m); bc_cols<I + 2, T>(u, c, m); }
+    else if constexpr (I < 16) { bc_cols1<I>(u + I, c, m); }
+}
+
+template <int N>
+__device__ __forceinline__ float row_get(float v)
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x150 + N, 0xf, 0xf, true));
+}
+template <int N>
+__device__ __forceinline__ double row_get(double v)
 {
     const long long b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_readlane((int)b, src);
-    const int hi = __builtin_amdgcn_readlane((int)(b >> 32), src);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, 0x150 + N, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), 0x150 + N, 0xf, 0xf, true);
     return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
 }
 
@@ -64,29 +373,26 @@ template <class T, int KT>
 struct ResLds {
     static constexpr int PS = 36;                         // row stride: 16-byte aligned rows, few bank conflicts
     static constexpr int NTR = 16 * (KT - 2);             // trailing rows / columns
-    // two panel buffers, used by alternate panels (a panel's factors are
-    // stored while the next panel is being factored):
-    static constexpr int pn_off = 0;                      // Pn [16 KT][PS]: panel rows; after B2 rows >= 32 hold -L21
+    // two panel buffers, used by alternate panels (a wavefront may copy the
+    // next panel's tiles while another still stores this one's factors):
+    static constexpr int pn_off = 0;                      // Pn [16 KT][PS]: panel rows; after B rows >= 32 hold -L21
     static constexpr int ub_off = pn_off + 16 * KT * PS;  // UbT [NTR][PS]: U block, one column per row
-    static constexpr int pv_off = ub_off + NTR * PS;      // pivots [32]
-    static constexpr int rp_off = pv_off + 32;            // their reciprocals [32]
+    static constexpr int rp_off = ub_off + NTR * PS;      // pivot reciprocals [32]
     static constexpr int buf_elems = rp_off + 32;
-    static constexpr int LTS = 36;                        // L11T row stride (16-byte aligned rows)
-    static constexpr int lt_off = 2 * buf_elems;          // L11 transposed [32][LTS]
-    static constexpr size_t bytes = sizeof(T) * (size_t)(lt_off + 32 * LTS);
+    static constexpr size_t bytes = sizeof(T) * (size_t)(2 * buf_elems);
 };
 
 template <class T>
-__device__ inline T buffer_load(__amdgpu_buffer_rsrc_t r, int off);
+__device__ inline T buffer_load(__amdgpu_buffer_rsrc_t r, int off, int soff = 0);
 template <>
-__device__ inline float buffer_load<float>(__amdgpu_buffer_rsrc_t r, int off)
+__device__ inline float buffer_load<float>(__amdgpu_buffer_rsrc_t r, int off, int soff)
 {
-    return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0));
+    return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, off, soff, 0));
 }
 template <>
-__device__ inline double buffer_load<double>(__amdgpu_buffer_rsrc_t r, int off)
+__device__ inline double buffer_load<double>(__amdgpu_buffer_rsrc_t r, int off, int soff)
 {
-    const auto v = __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0);
+    const auto v = __builtin_amdgcn_raw_buffer_load_b64(r, off, soff, 0);
     return __longlong_as_double((long long)(((unsigned long long)v[1] << 32) | v[0]));
 }
 
@@ -106,72 +412,91 @@ __device__ inline void buffer_store<double>(double v, __amdgpu_buffer_rsrc_t r, 
     __builtin_amdgcn_raw_buffer_store_b64(x, r, off, 0, 0);
 }
 
-// N values of a 16-byte aligned LDS row (float: 16-byte loads), from
-// element 4 * (FROM / 4) on; the rest of v is left as it is
-template <class T, int N>
-__device__ inline void lds_row_from(const T* p, T (&v)[N], int from)
+// 16 values of a 16-byte aligned LDS row
+__device__ inline void lds_get16(const float* p, float (&v)[16])
 {
-    if constexpr (sizeof(T) == 4) {
-        const float4* q = reinterpret_cast<const float4*>(p);
+    const float4* q = reinterpret_cast<const float4*>(p);
 #pragma unroll
-        for (int i = 0; i < N / 4; ++i) {
-            if (4 * i + 3 >= from) {
-                const float4 x = q[i];
-                v[4 * i] = x.x; v[4 * i + 1] = x.y; v[4 * i + 2] = x.z; v[4 * i + 3] = x.w;
-            }
-        }
-    } else {
-#pragma unroll
-        for (int c = 0; c < N; ++c)
-            if (c >= from) v[c] = p[c];
+    for (int i = 0; i < 4; ++i) {
+        const float4 x = q[i];
+        v[4 * i] = x.x; v[4 * i + 1] = x.y; v[4 * i + 2] = x.z; v[4 * i + 3] = x.w;
     }
 }
-template <int FROM, class T, int N>
-__device__ inline void lds_row(const T* p, T (&v)[N])
+__device__ inline void lds_get16(const double* p, double (&v)[16])
 {
-    lds_row_from<T, N>(p, v, FROM);
+    const double2* q = reinterpret_cast<const double2*>(p);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const double2 x = q[i];
+        v[2 * i] = x.x; v[2 * i + 1] = x.y;
+    }
 }
-template <int N>
-__device__ inline void lds_store_row(float* p, const float (&v)[N])
+__device__ inline void lds_get4(const float* p, float (&v)[4])
+{
+    const float4 x = *reinterpret_cast<const float4*>(p);
+    v[0] = x.x; v[1] = x.y; v[2] = x.z; v[3] = x.w;
+}
+__device__ inline void lds_get4(const double* p, double (&v)[4])
+{
+    const double2* q = reinterpret_cast<const double2*>(p);
+    const double2 x = q[0], y = q[1];
+    v[0] = x.x; v[1] = x.y; v[2] = y.x; v[3] = y.y;
+}
+__device__ inline void lds_put16(float* p, const float (&v)[16])
 {
     float4* q = reinterpret_cast<float4*>(p);
 #pragma unroll
-    for (int i = 0; i < N / 4; ++i) q[i] = make_float4(v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]);
+    for (int i = 0; i < 4; ++i) q[i] = make_float4(v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]);
 }
-template <int N>
-__device__ inline void lds_store_neg_row(float* p, const float (&v)[N])
+__device__ inline void lds_put16(double* p, const double (&v)[16])
 {
-    float4* q = reinterpret_cast<float4*>(p);
+    double2* q = reinterpret_cast<double2*>(p);
 #pragma unroll
-    for (int i = 0; i < N / 4; ++i) q[i] = make_float4(-v[4 * i], -v[4 * i + 1], -v[4 * i + 2], -v[4 * i + 3]);
+    for (int i = 0; i < 8; ++i) q[i] = make_double2(v[2 * i], v[2 * i + 1]);
 }
 
 __device__ inline float pivot_rcp(float v) { return __builtin_amdgcn_rcpf(v); }
 __device__ inline double pivot_rcp(double v) { return 1.0 / v; }
 
-// All ones when x < 0, else 0: one field extract of the sign bit.  Range
-// predicates are combined as sign masks of differences (ANDed), so no
-// per-element compare writes a scalar mask register.
+// all ones when x < 0, else 0
 __device__ inline int neg_mask(int x) { return __builtin_amdgcn_sbfe(x, 31, 1); }
-// the sign of v flipped where m is all ones
-__device__ inline float flip_sign(float v, int m) { return __int_as_float(__float_as_int(v) ^ (m & (int)0x80000000)); }
-__device__ inline double flip_sign(double v, int m)
+// The pivot of step N from the lane row's copy d of the diagonal block (row
+// `c` of it in lane c): boosted unless `plain`, kept in pr by lane N; returns
+// the reciprocal of the lane's own candidate (lane N's is the pivot's).
+template <int N, class T>
+__device__ __forceinline__ T sub_panel_pivot(const T (&d)[16], T& pr, int c, bool plain)
 {
-    const unsigned long long sb = (unsigned long long)((unsigned)m & 0x80000000u) << 32;
-    return __longlong_as_double((long long)((unsigned long long)__double_as_longlong(v) ^ sb));
+    const T thr = (T)1e-7, nv = (T)1e-4;
+    T piv = d[N];
+    if (!(fabs(piv) > thr || plain)) piv = piv < (T)0 ? -nv : nv;
+    pr = c == N ? piv : pr;
+    return pivot_rcp(piv);
 }
-// a where m is all ones, else b
-__device__ inline float pick(float a, float b, int m)
+// Steps N .. 15 of a 16-column sub-panel: own is the lane's row of L (ROWS) or
+// column of U, rl what sub_panel_pivot<N> returned.  d is left with L below
+// the diagonal and U above (ROWS; the diagonal itself is in pr).  The next
+// pivot's entry is updated first, and its chain (boost, reciprocal, broadcast)
+// runs under the rest of the step.
+template <int N, bool ROWS, class T>
+__device__ __forceinline__ void sub_panel_steps(T (&d)[16], T (&own)[16], T& pr, T rl, int c, bool plain)
 {
-    return __int_as_float((__float_as_int(a) & m) | (__float_as_int(b) & ~m));
+    asm volatile("" : "+v"(c));   // masks of lane numbers are made where they are used
+    const T rp = row_get<N>(rl);
+    const T l = c > N ? d[N] * rp : (T)0;
+    if constexpr (ROWS) own[N] = own[N] * rp;
+    if constexpr (N + 1 < 16) {
+        bc_self1<N>(d + N + 1, l);
+        // row N of d is not changed by this step, so the order of the two is free
+        if constexpr (ROWS) bc_rows<N, N + 1, T>(own, d, own[N]);
+        else bc_cols<N + 1, T>(own, l, own[N]);
+        const T rn = sub_panel_pivot<N + 1, T>(d, pr, c, plain);
+        if constexpr (ROWS) d[N] = c > N ? l : d[N];
+        if constexpr (sizeof(T) == 4) __builtin_amdgcn_sched_barrier(0);
+        bc_self<N, N + 2, T>(d, l);
+        sub_panel_steps<N + 1, ROWS, T>(d, own, pr, rn, c, plain);
+    }
 }
-__device__ inline double pick(double a, double b, int m)
-{
-    const long long x = __double_as_longlong(a), y = __double_as_longlong(b);
-    const unsigned lo = ((unsigned)x & (unsigned)m) | ((unsigned)y & ~(unsigned)m);
-    const unsigned hi = ((unsigned)(x >> 32) & (unsigned)m) | ((unsigned)(y >> 32) & ~(unsigned)m);
-    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
-}
+
 template <class T, int KT, int NW>
 __global__ __launch_bounds__(64 * NW) void band_factor_resident_kernel(T* __restrict__ B0, T* __restrict__ B1,
                                                                    const T* __restrict__ Bin, int k_all,
@@ -181,9 +506,10 @@ __global__ __launch_bounds__(64 * NW) void band_factor_resident_kernel(T* __rest
     using acc_t = typename MF::acc_t;
     using LY = ResLds<T, KT>;
     constexpr int PS = LY::PS, NTR = LY::NTR, NS = KT * KT, SPW = (NS + NW - 1) / NW, HR = 32 + NTR;
-    constexpr int NT = 64 * NW;         // threads
-    constexpr int UOFF = 64 * (NW / 2); // first thread of the U12 solves in B2
-    static_assert(NTR <= UOFF && UOFF + NTR <= NT, "B2 thread ranges");
+    constexpr int RW = (16 + NTR + 63) / 64;   // wavefronts of the L rows in B, and of the U columns
+    constexpr int UOFF = 64 * RW;              // first thread of the U columns
+    constexpr int UT = sizeof(T) == 4 ? 2 : 1; // tiles in flight in the update between sub-panels (registers)
+    static_assert(2 * RW <= NW, "B thread ranges");
     static_assert(SPW <= 32, "slot class masks are 32-bit");
     const FactorJob job = jobs[blockIdx.x];
     const int k = job.kb > 0 ? job.kb : k_all;
@@ -197,16 +523,11 @@ __global__ __launch_bounds__(64 * NW) void band_factor_resident_kernel(T* __rest
     T* const sm = reinterpret_cast<T*>(smem_raw);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // uniform: slot logic stays scalar
 
-    // rem = len - j0 is the number of partition rows left from panel row j0;
-    // entry (dr, dc) of the panel's window is stored iff this mask is set
-    auto inb = [&](int dr, int dc, int rem) {
-        return neg_mask((dr - rem) & (dc - rem) & (dr - dc - k - 1) & (dc - dr - k - 1));
-    };
     // Tile loads are buffer loads over the partition's storage: every element
     // is one unconditional load, and entries outside the band or the
     // partition use an offset past the end of the buffer, which reads zero.
     // (A register only ever written by loads needs no wait for an earlier
-    // load into it.)  Element (j0 + dr, j0 + dc) is at element offset
+    // load into it.)  rem = len - j0 is the number of partition rows left.  Element (j0 + dr, j0 + dc) is at element offset
     // ob + dir * (dc * 2k + dr) with ob = rel0 + dir * (j0 * (2k + 1) + k).
     // The band is read from Bin when given (the LU and UL factorizations of
     // one partition then share one unfactored copy) and the factors are
@@ -220,72 +541,84 @@ __global__ __launch_bounds__(64 * NW) void band_factor_resident_kernel(T* __rest
     // A(dr0 + l % 16, dc0 + row(l, q)), so for each register the 16 lanes of
     // a group read 16 consecutive rows of one column (one contiguous segment
     // per lane group).
-    auto load_tile = [&](acc_t& t, int ob, int rem, int dr0, int dc0, int lr, int lane) {
-        const int dr = dr0 + lr;
+    // A lane's first element of the tile with its lowest address at byte
+    // offset so is lp0 bytes above it, its row less its column is e0 more
+    // than the tile's, and each further element is one column step on.
+    // sk = dr0 - dc0 + k, rr = rem - dr0 (rows of the tile in the partition;
+    // a column past its end is past the end of the buffer).
+    constexpr int CS = sizeof(T) == 4 ? 1 : 4;       // columns between a lane's elements
+    const int so_rev = dir < 0 ? (15 * wm1 + 15) * (int)sizeof(T) : 0;
+    const int cstep = dir * CS * wm1 * (int)sizeof(T);
+    const int lr0 = threadIdx.x & 15, lc0 = MF::row(threadIdx.x & 63, 0);
+    const int lp0 = so_rev + dir * (lc0 * wm1 + lr0) * (int)sizeof(T), e0 = lr0 - lc0;
+    auto load_tile = [&](acc_t& t, int so, int sk, int rr) {
+        const int e = lr0 < rr ? e0 + sk : INT_MIN;
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const int dc = dc0 + MF::row(lane, q);
-            const int m = inb(dr, dc, rem);
-            const int off = (((ob + dir * (dc * wm1 + dr)) * (int)sizeof(T)) & m) | ~m;
-            t[q] = buffer_load<T>(rsrc_in, off);
-        }
+        for (int q = 0; q < 4; ++q)
+            t[q] = buffer_load<T>(rsrc_in, (unsigned)(e - CS * q) <= (unsigned)wm1 ? lp0 + so + q * cstep : -1);
     };
-    // factors of panel pp from panel buffer bq: its 32 columns (rows 0 .. HR-1:
-    // L, D, U' of the diagonal block and L21) and its 32 U' rows, coalesced
-    // (values are gathered from LDS first and stored afterwards, so the LDS
-    // reads overlap instead of each store waiting for its own read).  The
-    // stores are unconditional buffer stores: entries outside the band get
-    // an offset past the end of the buffer and are dropped, so every panel
-    // issues the same number of stores (pp < 0: none land).
-    // Stored by wavefronts 1 .. NW-1 (st = thread index - 64): wavefront 0
-    // factors the next diagonal block meanwhile.
-    constexpr int NTS = NT - 64;
-    auto store_panel = [&](int64_t pp, const T* bq, int st) {
-        constexpr int N1 = (32 * HR + NTS - 1) / NTS, N2 = (32 * NTR + NTS - 1) / NTS;
-        const int64_t pj0 = 32 * max(pp, (int64_t)0);
+    // so of the tile at (dr0, dc0) of the panel whose window begins at element ob
+    auto tile_off = [&](int ob, int dr0, int dc0) {
+        return (ob + dir * (dc0 * wm1 + dr0)) * (int)sizeof(T) - so_rev;
+    };
+    // Factors of panel pp from panel buffer bq: its 32 columns (rows 0 .. HR-1:
+    // L, D, U' of the diagonal block and L21), a column and 64 rows at a time,
+    // and its 32 U' rows, two columns at a time.  Lanes run up the addresses;
+    // entries outside the band get an offset past the end of the buffer and
+    // are dropped.
+    auto store_panel = [&](int64_t pp, const T* bq, int lane) {
+        constexpr int NG = (HR + 63) / 64;
+        const int64_t pj0 = 32 * pp;
         const int obq = rel0 + dir * (int)(pj0 * w + k);
-        const int prem = pp < 0 ? 0 : (int)min(len - pj0, (int64_t)(1 << 30));
+        const int prem = (int)min(len - pj0, (int64_t)(1 << 30));
         const int pnb = min(32, prem);
         const T* qPn = bq + LY::pn_off;
         const T* qUb = bq + LY::ub_off;
         const T* qrp = bq + LY::rp_off;   // pivot reciprocals (0 past the partition's end)
-        T v1[N1], v2[N2];
-        int o1[N1], o2[N2];
+        const int rl = dir > 0 ? lane : 63 - lane;
+        const T f0 = qrp[rl & 31];
+#pragma unroll 1
+        for (int c = wave; c < pnb; c += NW) {
+            T v[NG];
 #pragma unroll
-        for (int i = 0; i < N1; ++i) {
-            const int e = st + NTS * i;
-            const int c = e / HR, r = e - c * HR;
-            const int ok = neg_mask((e - 32 * HR) & (c - pnb) & (r - prem) & (r - c - k - 1) & (c - r - k - 1));
-            const int lrow = ~neg_mask(r - 32);   // L21 rows, kept negated in LDS
-            const int upper = neg_mask(r - c);    // U' of the diagonal block: scaled by 1 / pivot
-            const T v = qPn[(r * PS + c) & ok];
-            const T f = qrp[r & ~lrow & 31];
-            v1[i] = flip_sign(v * pick(f, (T)1, upper), lrow);
-            o1[i] = (((obq + dir * (c * wm1 + r)) * (int)sizeof(T)) & ok) | ~ok;
+            for (int g = 0; g < NG; ++g) v[g] = qPn[min(64 * g + rl, HR - 1) * PS + c];
+            // U' of the diagonal block is scaled by 1 / pivot; L21 rows are
+            // kept negated in LDS
+            v[0] = rl >= 32 ? -v[0] : (rl < c ? v[0] * f0 : v[0]);
+            const int lo = max(c - k, 0), top = min(min(HR, prem), c + k + 1);   // rows [lo, top) are stored
+            const int oc = (obq + dir * (c * wm1 + rl)) * (int)sizeof(T);
+#pragma unroll
+            for (int g = 0; g < NG; ++g) {
+                const bool in = (unsigned)(rl + 64 * g - lo) < (unsigned)(top - lo);
+                buffer_store<T>(g == 0 ? v[g] : -v[g], rsrc, in ? oc + dir * 64 * g * (int)sizeof(T) : -1);
+            }
         }
+        const int half = lane >> 5, um = dir > 0 ? lane & 31 : 31 - (lane & 31);
+        const T fu = qrp[um];
+        const int ul = (obq + dir * ((32 + half) * wm1 + um)) * (int)sizeof(T);
+        const int ctop = min(min(NTR, prem - 32), k);
+#pragma unroll 1
+        for (int c0 = 2 * wave; c0 < ctop; c0 += 8 * NW) {
+            T v[4];
 #pragma unroll
-        for (int i = 0; i < N2; ++i) {
-            const int e = st + NTS * i;
-            const int cc = e >> 5, m = e & 31;
-            const int ok = neg_mask((e - 32 * NTR) & (m - pnb) & (32 + cc - prem) & (32 + cc - m - k - 1));
-            v2[i] = qUb[(cc * PS + m) & ok] * qrp[m];
-            o2[i] = (((obq + dir * ((32 + cc) * wm1 + m)) * (int)sizeof(T)) & ok) | ~ok;
+            for (int i = 0; i < 4; ++i) v[i] = qUb[min(c0 + half + 2 * NW * i, NTR - 1) * PS + um];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int cc = c0 + half + 2 * NW * i;
+                const bool in = um < pnb && cc < ctop && um >= 32 + cc - k;
+                buffer_store<T>(v[i] * fu, rsrc, in ? ul + dir * (c0 + 2 * NW * i) * wm1 * (int)sizeof(T) : -1);
+            }
         }
-#pragma unroll
-        for (int i = 0; i < N1; ++i) buffer_store<T>(v1[i], rsrc, o1[i]);
-#pragma unroll
-        for (int i = 0; i < N2; ++i) buffer_store<T>(v2[i], rsrc, o2[i]);
     };
 
     acc_t acc[SPW];
     {
-        const int lane = threadIdx.x & 63;
         const int ob = rel0 + dir * k;
         const int rem = (int)min(len, (int64_t)(1 << 30));
 #pragma unroll
         for (int j = 0; j < SPW; ++j) {
-            const int s = wave + NW * j;
-            if (s < NS) load_tile(acc[j], ob, rem, 16 * (s / KT), 16 * (s % KT), lane & 15, lane);
+            const int s = wave + NW * j, dr0 = 16 * (s / KT), dc0 = 16 * (s % KT);
+            if (s < NS) load_tile(acc[j], tile_off(ob, dr0, dc0), dr0 - dc0 + k, rem - dr0);
         }
     }
 
@@ -302,22 +635,24 @@ __global__ __launch_bounds__(64 * NW) void band_factor_resident_kernel(T* __rest
         T* bcur = sm + zoff + cur * LY::buf_elems;
         T* Pn = bcur + LY::pn_off;
         T* UbT = bcur + LY::ub_off;
-        T* pivs = bcur + LY::pv_off;
         T* rpiv = bcur + LY::rp_off;
-        T* L11T = sm + zoff + LY::lt_off;
         const int64_t j0 = 32 * p;
         const int rem = (int)min(len - j0, (int64_t)(1 << 30));
         const int nb = min(32, rem);
         const int sh = (int)((2 * p) % KT);
         const int obp = rel0 + dir * (int)(j0 * w + k);
-        // Slot bookkeeping, lane-parallel: lane j holds the rotated tile
-        // coordinates (rho, gam) of this wavefront's slot j (s = wave + NW j,
-        // clamped to NS - 1 past the last slot), and three ballots give the
-        // slot classes: panel column (gam < 2), U row (rho < 2 <= gam) and
-        // trailing (both >= 2).  Each unrolled slot step then costs a mask bit
-        // test and one readlane instead of its own scalar index arithmetic.
-        unsigned pm, um, tm, dm;
-        int rg;
+        // Slot bookkeeping, lane-parallel: lane j holds, for slot j of this
+        // wavefront (s = wave + NW j, clamped to NS - 1 past the last slot)
+        // with rotated tile coordinates (rl, gl), the LDS offset it is copied
+        // to, the place of the tile it loads next and the LDS offsets of its
+        // operands; three ballots give the slot classes: panel column
+        // (gl < 2), U row (rl < 2 <= gl) and trailing (both >= 2).  Each
+        // unrolled slot step then costs a mask bit test and a few readlanes
+        // instead of its own scalar index arithmetic: the panel loop has to
+        // stay well inside the 64 KiB instruction cache that two compute
+        // units share.
+        unsigned pm, um, tm;
+        int cpo, lso, lsk, lrr, mao, mbo;
         {
             const int sl = min(wave + NW * lane, NS - 1);
             int rl = sl / KT - sh, gl = sl % KT - sh;
@@ -327,276 +662,190 @@ __global__ __launch_bounds__(64 * NW) void band_factor_resident_kernel(T* __rest
             pm = (unsigned)__builtin_amdgcn_ballot_w64(okl && gl < 2);
             um = (unsigned)__builtin_amdgcn_ballot_w64(okl && gl >= 2 && rl < 2);
             tm = (unsigned)__builtin_amdgcn_ballot_w64(okl && gl >= 2 && rl >= 2);
-            dm = (unsigned)__builtin_amdgcn_ballot_w64(okl && gl < 2 && rl < 2);   // diagonal block
-            rg = rl | (gl << 8);
+            mao = 16 * PS * rl;
+            mbo = LY::ub_off + 16 * PS * (gl - 2);
+            cpo = gl < 2 ? mao + 16 * gl : mbo + 16 * rl;
+            const int dr0 = 16 * (rl < 2 ? rl + KT : rl), dc0 = 16 * (gl < 2 ? gl + KT : gl);
+            lso = tile_off(obp, dr0, dc0);
+            lsk = dr0 - dc0 + k;
+            lrr = rem - dr0;
         }
-        // rho and gam of slot j (j a compile-time constant)
-        auto slot_rho = [&](int j) { return __builtin_amdgcn_readlane(rg, j) & 0xff; };
-        auto slot_gam = [&](int j) { return __builtin_amdgcn_readlane(rg, j) >> 8; };
+        auto of_slot = [&](int v, int j) { return __builtin_amdgcn_readlane(v, j); };   // j a compile-time constant
 
-        // Every load and store of the previous panel has long completed (B2
-        // and C ran since); saying so with an explicit wait clears the
-        // compiler's record of loads pending across the loop back-edge, which
-        // would otherwise make each slot below wait for the loads just issued
-        // by the slots before it (vmcnt bits [3:0] and [15:14] = 0, expcnt and
-        // lgkmcnt at their maxima).
-        __builtin_amdgcn_s_waitcnt((0x7 << 4) | (0xF << 8));
-        // A0. the diagonal block's four tiles to LDS: B1 needs nothing else,
-        //     so wavefront 0 factors it while the others finish phase A.
+        // A. the leaving tiles to LDS, then their slots load the entering
+        //    tiles.  (All copies to LDS come first: reading a slot that may
+        //    still be loading waits for every load issued before it.)
 #pragma unroll
         for (int j = 0; j < SPW; ++j) {
-            if ((dm >> j) & 1) {
-                const int rho = slot_rho(j), gam = slot_gam(j);
+            if ((pm >> j) & 1) {
+                T* const pt = bcur + of_slot(cpo, j) + lr * PS;
+                if constexpr (sizeof(T) == 4) {   // four consecutive columns
+                    *reinterpret_cast<acc_t*>(pt + 4 * lg) = acc[j];
+                } else {
 #pragma unroll
-                for (int q = 0; q < 4; ++q) Pn[(16 * rho + lr) * PS + 16 * gam + MF::row(lane, q)] = acc[j][q];
-            }
-        }
-        lds_barrier();
-
-        // B1. LU of the diagonal block (wavefront 0), row r in lane r (lanes
-        //     32..63 mirror).  It writes rows 0..31 of Pn, the pivots and L11^T
-        //     only, which the rest of phase A does not touch.
-        //     Straight-line code (no branch per column), so the scheduler can
-        //     run ahead: a lane that must not change gets multiplier 0, and
-        //     columns past the partition's end (last panel) get reciprocal 0,
-        //     which makes their steps exact no-ops.
-        if (wave == 0) {
-            const int r = lane & 31;
-            T row[32];
-            T pr = (T)0;   // this lane's pivot
-#pragma unroll
-            for (int c = 0; c < 32; ++c) row[c] = Pn[r * PS + c];
-#pragma unroll
-            for (int jj = 0; jj < 32; ++jj) {
-                T piv = lane_bcast(row[jj], jj);
-                if (job.boost && (jj + 1 < rem || job.boost_last)) piv = boost_pivot(piv);
-                const T rp = jj < nb ? pivot_rcp(piv) : (T)0;
-                const T l = r > jj ? row[jj] * rp : (T)0;
-                pr = r == jj ? piv : pr;
-#pragma unroll
-                for (int c = jj + 1; c < 32; ++c) row[c] -= l * lane_bcast(row[c], jj);   // pivot row, before any update
-                row[jj] = r > jj ? l : (r == jj ? piv : row[jj]);
-            }
-            if (lane < 32) {
-                pivs[r] = pr;
-                rpiv[r] = r < nb ? pivot_rcp(pr) : (T)0;
-#pragma unroll
-                for (int c = 0; c < 32; ++c) {
-                    Pn[r * PS + c] = row[c];
-                    if (c < r) L11T[c * LY::LTS + r] = row[c];
+                    for (int q = 0; q < 4; ++q) pt[MF::row(lane, q)] = acc[j][q];
                 }
-            }
-        }
-        // A. the other leaving tiles to LDS, then their slots load the entering
-        //    tiles, then the previous panel's factors go out: every global
-        //    access of the panel is issued here, so loads and stores drain
-        //    during B2 and C before the next panel needs them.  (All copies to
-        //    LDS come first: reading a slot that may still be loading waits for
-        //    every load issued before it.)
-#pragma unroll
-        for (int j = 0; j < SPW; ++j) {
-            if (((pm & ~dm) >> j) & 1) {
-                const int rho = slot_rho(j), gam = slot_gam(j);
-#pragma unroll
-                for (int q = 0; q < 4; ++q) Pn[(16 * rho + lr) * PS + 16 * gam + MF::row(lane, q)] = acc[j][q];
             } else if ((um >> j) & 1) {
-                const int rho = slot_rho(j), gam = slot_gam(j);
+                T* const pt = bcur + of_slot(cpo, j) + lr;
 #pragma unroll
-                for (int q = 0; q < 4; ++q) UbT[(16 * (gam - 2) + MF::row(lane, q)) * PS + 16 * rho + lr] = acc[j][q];
+                for (int q = 0; q < 4; ++q) pt[MF::row(lane, q) * PS] = acc[j][q];
             }
         }
-#pragma unroll
-        for (int j = 0; j < SPW; ++j) {
-            if (((pm | um) >> j) & 1) {
-                const int rho = slot_rho(j), gam = slot_gam(j);
-                const int rn = rho < 2 ? rho + KT - 2 : rho - 2;
-                const int cn = gam < 2 ? gam + KT - 2 : gam - 2;
-                load_tile(acc[j], obp, rem, 32 + 16 * rn, 32 + 16 * cn, lr, lane);
-            }
-        }
-        if (wave > 0) store_panel(p - 1, sm + zoff + (1 - cur) * LY::buf_elems, tid - 64);
         lds_barrier();
+#pragma unroll
+        for (int j = 0; j < SPW; ++j)
+            if (((pm | um) >> j) & 1) load_tile(acc[j], of_slot(lso, j), of_slot(lsk, j), of_slot(lrr, j));
 
-        // B2. L21 rows (stored negated: the trailing update adds) and U12 columns
-        if constexpr (sizeof(T) == 4) {
-            // FP32, by halves: columns 0..15 of L21 = A21 U11^-1 (rows 0..15 of
-            // U12 = L11^-1 A12) by substitution; their contribution to the
-            // other half (A21_b -= L21_a U11_ab, A12_b -= L11_ba U12_a) on the
-            // matrix cores; then the other half by substitution.  The U11
-            // (L11^T) rows come in 16-byte loads one step ahead of their use.
-            if (tid < NTR) {
-                const int t = tid;
-                T a[16], cur[16], nxt[16];
-                lds_row<0>(Pn + (32 + t) * PS, a);
-                lds_row<1>(Pn, cur);
+        // B. the two sub-panels (columns O .. O + 15).  Threads 0 .. 15 + NTR - O
+        //    hold rows 16 + O .. of the panel, threads UOFF .. the columns 16 + O ..
+        //    (the first 16 of sub-panel 0 are the panel's own columns 16 .. 31,
+        //    in Pn; the rest UbT).
+        const int boosted = job.boost ? (job.boost_last ? 32 : min(32, rem - 1)) : 0;
+#pragma unroll 1
+        for (int O = 0; O < 32; O += 16) {
+            int c16 = lane & 15;
+            asm volatile("" : "+v"(c16));
+            T d[16], own[16], pr = (T)0;
+            lds_get16(Pn + (O + c16) * PS + O, d);
+            const bool urow = wave < RW;
+            const int t = urow ? tid : tid - UOFF;         // row 16 + O + t, or column t
+            const bool on = t < 16 + NTR - O;
+            const bool incol = O == 0 && !urow && t < 16;  // a column of the panel itself
+            T* const mine = urow ? Pn + (16 + O + t) * PS + O : UbT + (t - (16 - O)) * PS + O;
+            if (incol) {
 #pragma unroll
-                for (int jj = 0; jj < 16; ++jj) {   // rpiv = 0 past the partition's end
-                    if (jj < 15) lds_row_from<T>(Pn + (jj + 1) * PS, nxt, jj + 2);
-                    const T l = a[jj] * rpiv[jj];
-                    a[jj] = l;
+                for (int i = 0; i < 16; ++i) own[i] = Pn[i * PS + 16 + t];
+            } else if (on) {
+                lds_get16(mine, own);
+            } else {
 #pragma unroll
-                    for (int c = jj + 1; c < 16; ++c) a[c] -= l * cur[c];
+                for (int i = 0; i < 16; ++i) own[i] = (T)0;
+            }
+            lds_barrier();   // every copy of the diagonal block is read before it is overwritten
+            const bool live = O + c16 < nb, plain = O + c16 >= boosted;
+            if (nb < 32) {   // a unit pivot makes the steps past the partition's end exact no-ops
+                int cd = live ? -1 : c16;
+                asm volatile("" : "+v"(cd));
 #pragma unroll
-                    for (int c = 0; c < 16; ++c) cur[c] = nxt[c];
+                for (int i = 0; i < 16; ++i) d[i] = i == cd ? (T)1 : d[i];
+            }
+            if (wave < 2 * RW) {
+                const T rl = sub_panel_pivot<0, T>(d, pr, c16, plain);
+                if (urow) sub_panel_steps<0, true, T>(d, own, pr, rl, c16, plain);
+                else sub_panel_steps<0, false, T>(d, own, pr, rl, c16, plain);
+            }
+            if (incol) {
+#pragma unroll
+                for (int i = 0; i < 16; ++i) Pn[i * PS + 16 + t] = own[i];
+            } else if (on) {
+                if (urow && 16 + O + t >= 32) {            // L21 is kept negated: the trailing update adds
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) own[i] = -own[i];
                 }
-                lds_store_neg_row(Pn + (32 + t) * PS, a);
-            } else if (tid >= UOFF && tid < UOFF + NTR) {
-                const int cc = tid - UOFF;
-                T u[16], cur[16], nxt[16];
-                lds_row<0>(UbT + cc * PS, u);
-                lds_row<1>(L11T, cur);
-#pragma unroll
-                for (int jj = 0; jj < 15; ++jj) {   // u[jj] = 0 past the partition's end
-                    if (jj < 14) lds_row_from<T>(L11T + (jj + 1) * LY::LTS, nxt, jj + 2);
-                    const T uj = u[jj];
-#pragma unroll
-                    for (int m = jj + 1; m < 16; ++m) u[m] -= cur[m] * uj;
-#pragma unroll
-                    for (int m = 0; m < 16; ++m) cur[m] = nxt[m];
-                }
-                lds_store_row(UbT + cc * PS, u);
+                lds_put16(mine, own);
+            }
+            if (tid < 16) {
+                lds_put16(Pn + (O + tid) * PS + O, d);
+                Pn[(O + tid) * PS + O + tid] = pr;
+                rpiv[O + tid] = live ? pivot_rcp(pr) : (T)0;
             }
             lds_barrier();
-            {
-                // 16 x 16 tiles: KT-2 of L21's rows (A = the stored -L21_a,
-                // B = U11 rows 0..15, columns 16..31) and KT-2 of U12's
-                // columns (A = -U12_a^T, B = L11^T rows 0..15, columns 16..31)
-                const int g = lane >> 4, c16 = lane & 15;
-                for (int f = wave; f < 2 * (KT - 2); f += NW) {
-                    const bool lside = f < KT - 2;
-                    const int r0 = lside ? 32 + 16 * f : 16 * (f - (KT - 2));
-                    T* const rows = lside ? Pn : UbT;
-                    const T* const bm = lside ? Pn : L11T;
-                    const int bs = lside ? PS : LY::LTS;
-                    acc_t acc;
+            if (O == 0) {
+                // columns 16 .. 31 of the rows below (A = -L_a, B = rows 0 .. 15 of
+                // U, columns 16 .. 31), and rows 16 .. 31 of the columns right
+                // (A = -U_a^T, B = L_ba^T), 16 x 16 tiles
+                const int g = lane >> 4;
+#pragma unroll 1
+                for (int f0 = wave; f0 < 2 * KT - 3; f0 += UT * NW) {
+                    T* at[UT];
+                    acc_t ac[UT];
+                    T av[UT][4], bv[UT][4];
 #pragma unroll
-                    for (int q = 0; q < 4; ++q) acc[q] = rows[(r0 + MF::row(lane, q)) * PS + 16 + c16];
+                    for (int i = 0; i < UT; ++i) {
+                        const int f = min(f0 + NW * i, 2 * KT - 4);
+                        const bool lside = f < KT - 1;
+                        const T* const rows = lside ? Pn + (16 + 16 * f) * PS : UbT + 16 * (f - (KT - 1)) * PS;
+                        const bool neg = f == 0 || !lside;   // operands not kept negated
+                        at[i] = const_cast<T*>(rows) + MF::row(lane, 0) * PS + 16 + c16;
 #pragma unroll
-                    for (int st = 0; st < 4; ++st) {
-                        const T av = rows[(r0 + c16) * PS + 4 * st + g];
-                        const T bv = bm[(4 * st + g) * bs + 16 + c16];
-                        acc = MF::mma(lside ? av : -av, bv, acc);
+                        for (int q = 0; q < 4; ++q) ac[i][q] = at[i][CS * q * PS];
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) {
+                            const T x = rows[c16 * PS + 4 * q + g];
+                            av[i][q] = neg ? -x : x;
+                            bv[i][q] = lside ? Pn[(4 * q + g) * PS + 16 + c16] : Pn[(16 + c16) * PS + 4 * q + g];
+                        }
                     }
 #pragma unroll
-                    for (int q = 0; q < 4; ++q) rows[(r0 + MF::row(lane, q)) * PS + 16 + c16] = acc[q];
+                    for (int q = 0; q < 4; ++q)
+#pragma unroll
+                        for (int i = 0; i < UT; ++i) ac[i] = MF::mma(av[i][q], bv[i][q], ac[i]);
+#pragma unroll
+                    for (int i = 0; i < UT; ++i)
+                        if (f0 + NW * i < 2 * KT - 3) {
+#pragma unroll
+                            for (int q = 0; q < 4; ++q) at[i][CS * q * PS] = ac[i][q];
+                        }
                 }
+                lds_barrier();
             }
-            lds_barrier();
-            if (tid < NTR) {
-                const int t = tid;
-                T a[16], cur[16], nxt[16];   // columns 16..31
-                lds_row<0>(Pn + (32 + t) * PS + 16, a);
-                lds_row<1>(Pn + 16 * PS + 16, cur);
-#pragma unroll
-                for (int jj = 0; jj < 16; ++jj) {
-                    if (jj < 15) lds_row_from<T>(Pn + (17 + jj) * PS + 16, nxt, jj + 2);
-                    const T l = a[jj] * rpiv[16 + jj];
-                    a[jj] = l;
-#pragma unroll
-                    for (int c = jj + 1; c < 16; ++c) a[c] -= l * cur[c];
-#pragma unroll
-                    for (int c = 0; c < 16; ++c) cur[c] = nxt[c];
-                }
-                lds_store_neg_row(Pn + (32 + t) * PS + 16, a);
-            } else if (tid >= UOFF && tid < UOFF + NTR) {
-                const int cc = tid - UOFF;
-                T u[16], cur[16], nxt[16];   // rows 16..31
-                lds_row<0>(UbT + cc * PS + 16, u);
-                lds_row<1>(L11T + 16 * LY::LTS + 16, cur);
-#pragma unroll
-                for (int jj = 0; jj < 15; ++jj) {
-                    if (jj < 14) lds_row_from<T>(L11T + (17 + jj) * LY::LTS + 16, nxt, jj + 2);
-                    const T uj = u[jj];
-#pragma unroll
-                    for (int m = jj + 1; m < 16; ++m) u[m] -= cur[m] * uj;
-#pragma unroll
-                    for (int m = 0; m < 16; ++m) cur[m] = nxt[m];
-                }
-                lds_store_row(UbT + cc * PS + 16, u);
-            }
-        } else if (tid < NTR) {
-            const int t = tid;
-            T a[32];
-#pragma unroll
-            for (int c = 0; c < 32; ++c) a[c] = Pn[(32 + t) * PS + c];
-#pragma unroll
-            for (int jj = 0; jj < 32; ++jj) {   // rpiv = 0 past the partition's end
-                const T l = a[jj] * rpiv[jj];
-                a[jj] = l;
-#pragma unroll
-                for (int c = jj + 1; c < 32; ++c) a[c] -= l * Pn[jj * PS + c];
-            }
-#pragma unroll
-            for (int c = 0; c < 32; ++c) Pn[(32 + t) * PS + c] = -a[c];
-        } else if (tid >= UOFF && tid < UOFF + NTR) {
-            const int cc = tid - UOFF;
-            T u[32];
-#pragma unroll
-            for (int m = 0; m < 32; ++m) u[m] = UbT[cc * PS + m];
-#pragma unroll
-            for (int jj = 0; jj < 31; ++jj) {   // u[jj] = 0 past the partition's end
-                const T uj = u[jj];
-#pragma unroll
-                for (int m = jj + 1; m < 32; ++m) u[m] -= L11T[jj * LY::LTS + m] * uj;
-            }
-#pragma unroll
-            for (int m = 0; m < 32; ++m) UbT[cc * PS + m] = u[m];
         }
-        lds_barrier();
 
-        // C. trailing update on the matrix cores.  The next panel writes the
-        //    other buffer, so no barrier is needed after this phase.
-        if constexpr (sizeof(T) == 4) {
-            // FP32: each slot's operands are two 16-byte rows (lane group lg
-            // takes k = 8 lg .. 8 lg + 7), fetched one slot ahead of the slot
-            // being multiplied.  The fetches are unconditional: for a slot
-            // that is not updated (panel rows or columns; s >= NS reads slot
-            // NS - 1) the addresses still fall inside this panel buffer (rows
-            // 16 rho + lr < 16 KT of Pn, or rows of UbT at most 32 before it,
-            // which are rows of Pn), and the values go unused.
-            auto fetch = [&](int j, float4 (&o)[4]) {
-                const int rho = slot_rho(j), gam = slot_gam(j);
-                const float4* ap = reinterpret_cast<const float4*>(Pn + (16 * rho + lr) * PS + 8 * lg);
-                const float4* bp = reinterpret_cast<const float4*>(UbT + (16 * (gam - 2) + lr) * PS + 8 * lg);
-                o[0] = ap[0]; o[1] = ap[1]; o[2] = bp[0]; o[3] = bp[1];
-            };
-            float4 op[4], nx[4];
-            fetch(0, op);
-#pragma unroll
-            for (int j = 0; j < SPW; ++j) {
-                if (j + 1 < SPW) fetch(j + 1, nx);
-                if ((tm >> j) & 1) {
-                    const float av[8] = {op[0].x, op[0].y, op[0].z, op[0].w, op[1].x, op[1].y, op[1].z, op[1].w};
-                    const float bv[8] = {op[2].x, op[2].y, op[2].z, op[2].w, op[3].x, op[3].y, op[3].z, op[3].w};
-#pragma unroll
-                    // transposed tiles: acc^T += U12^T (-L21)^T
-                    for (int q = 0; q < 8; ++q) acc[j] = MF::mma(bv[q], av[q], acc[j]);
-                }
-#pragma unroll
-                for (int i = 0; i < 4; ++i) op[i] = nx[i];
+        // C. trailing update on the matrix cores and the panel's factors out.
+        //    The next panel writes the other buffer, so no barrier is needed
+        //    after this phase.
+        // Every tile load of this panel has long completed (B ran since);
+        // saying so with an explicit wait before the stores are issued clears
+        // the compiler's record of loads pending across the loop back-edge,
+        // which would otherwise make each slot of the next phase A wait for
+        // the loads just issued by the slots before it, and for the stores
+        // (vmcnt bits [3:0] and [15:14] = 0, expcnt and lgkmcnt at their
+        // maxima).
+        __builtin_amdgcn_s_waitcnt((0x7 << 4) | (0xF << 8));
+        if (wave >= NW / 2) store_panel(p, bcur, lane);
+        if (tm) {
+            // Each slot's operands are two rows of 8 values (lane group lg
+            // takes k = 8 lg .. 8 lg + 7), in two halves; each half of the
+            // next trailing slot's is fetched while the other half of this
+            // one's is multiplied.  Lane j holds the operand offsets of the
+            // slot after trailing slot j (its own again for the last), so
+            // that both are in one basic block.
+            const T* const al = bcur + lr * PS + 8 * lg;
+            const unsigned after = tm & (~1u << (lane & 31));
+            const int nj = 4 * (after ? __builtin_ctz(after) : 31 - __builtin_clz(tm)), first = __builtin_ctz(tm);
+            const int nma = __builtin_amdgcn_ds_bpermute(nj, mao), nmb = __builtin_amdgcn_ds_bpermute(nj, mbo);
+            T a0[4], b0[4], a1[4], b1[4];
+            {
+                const T* const ap = al + __builtin_amdgcn_readlane(mao, first);
+                const T* const bp = al + __builtin_amdgcn_readlane(mbo, first);
+                lds_get4(ap, a0); lds_get4(bp, b0); lds_get4(ap + 4, a1); lds_get4(bp + 4, b1);
             }
-        } else {
 #pragma unroll
             for (int j = 0; j < SPW; ++j) {
                 if ((tm >> j) & 1) {
-                    const int rho = slot_rho(j), gam = slot_gam(j);
-                    const T* ap = Pn + (16 * rho + lr) * PS + 8 * lg;
-                    const T* bp = UbT + (16 * (gam - 2) + lr) * PS + 8 * lg;
-                    T av[8], bv[8];
+                    const T* const ap = al + of_slot(nma, j);
+                    const T* const bp = al + of_slot(nmb, j);
+                    // transposed tiles: acc^T += U12^T (-L21)^T
 #pragma unroll
-                    for (int q = 0; q < 8; ++q) { av[q] = ap[q]; bv[q] = bp[q]; }
+                    for (int q = 0; q < 4; ++q) acc[j] = MF::mma(b0[q], a0[q], acc[j]);
+                    __builtin_amdgcn_sched_barrier(0);
+                    lds_get4(ap, a0); lds_get4(bp, b0);
+                    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                    for (int q = 0; q < 8; ++q) acc[j] = MF::mma(bv[q], av[q], acc[j]);
+                    for (int q = 0; q < 4; ++q) acc[j] = MF::mma(b1[q], a1[q], acc[j]);
+                    __builtin_amdgcn_sched_barrier(0);
+                    lds_get4(ap + 4, a1); lds_get4(bp + 4, b1);
                 }
             }
         }
+        if (wave < NW / 2) store_panel(p, bcur, lane);
     }
-    if (npan > 0 && wave > 0) store_panel(npan - 1, sm + ((npan - 1) & 1) * LY::buf_elems, (int)threadIdx.x - 64);
 }
 
-// Wavefronts per workgroup: the window's tiles are spread over them, so more
-// wavefronts leave each more registers for the panel phases (and more
-// latency hiding), as long as the accumulators still fit.
+// Wavefronts per workgroup.  Sixteen leave 128 registers each: equal at
+// k = 50 (2.77 against 2.79 ms of setup, n = 200000), faster at k = 120 (LU
+// 9.1 against 9.6 ms, n = 400000), but from k = 180 the tiles and the panel
+// rows no longer fit and spill (9.8 against 9.4 ms at k = 200).
 template <class T, int KT>
 constexpr int resident_waves() { return 8; }
 
