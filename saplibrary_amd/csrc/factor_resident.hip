@@ -842,10 +842,10 @@ __global__ __launch_bounds__(64 * NW) void band_factor_resident_kernel(T* __rest
     }
 }
 
-// Wavefronts per workgroup.  Sixteen leave 128 registers each: equal at
-// k = 50 (2.77 against 2.79 ms of setup, n = 200000), faster at k = 120 (LU
-// 9.1 against 9.6 ms, n = 400000), but from k = 180 the tiles and the panel
-// rows no longer fit and spill (9.8 against 9.4 ms at k = 200).
+// Wavefronts per workgroup.  Sixteen leave 128 registers each: no faster where
+// the tiles fit (k = 50: 2.59 against 2.58 ms for LU and UL, n = 200000), and
+// from k = 100 they spill (k = 120: 8.97 against 8.41 ms, k = 200: 10.4
+// against 8.28).
 template <class T, int KT>
 constexpr int resident_waves() { return 8; }
 
