@@ -127,9 +127,9 @@ __global__ __launch_bounds__(256) void band_factor_kernel(T* __restrict__ B0, T*
 }
 
 // ---------------------------------------------------------------------------
-// MFMA variant of the blocked banded LU (32-column panels), for the bands the
-// register-resident kernel does not take, up to k = 480 (256 or 512
-// threads, one panel row each).  Per panel:
+// MFMA variant of the blocked banded LU (32-column panels) for the FP64 bands
+// whose panel is too large for the LDS of the other blocked kernel, k = 225
+// to 480 (512 threads, one panel row each).  Per panel:
 //   1. every thread holds one row of the (32 + k) x 32 panel in
 //      registers and the panel is factored column by column (boosting at
 //      pivot time); the pivot row is broadcast through LDS, one barrier per
@@ -139,30 +139,13 @@ __global__ __launch_bounds__(256) void band_factor_kernel(T* __restrict__ B0, T*
 //      one column step behind (multipliers shared through LDS);
 //   3. the k x k trailing window in global memory (L2) receives the rank-32
 //      update -L_below * U_right on the matrix cores
-//      (v_mfma_f32_32x32x2f32, or v_mfma_f64_16x16x4f64 in FP64), tiles
-//      held transposed so that their loads and stores run along columns,
+//      (v_mfma_f64_16x16x4f64), tiles held transposed so that their loads and stores run along columns,
 //      four tiles per wavefront in flight; -L_below comes from LDS or, for
 //      the widest FP64 bands, from the band itself.
 // Factors are written as L (unit), D, U' (divided), like the LDS variant.
 // ---------------------------------------------------------------------------
 template <class T>
 struct Mfma;
-
-template <>
-struct Mfma<float> {
-    static constexpr int TILE = 32, KSTEP = 2, NACC = 16;
-    typedef float acc_t __attribute__((ext_vector_type(16)));
-    __device__ static inline acc_t mma(float a, float b, acc_t c)
-    {
-        return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
-    }
-    // accumulator register r of lane l holds D[row(l, r)][col(l)]
-    __device__ static inline int row(int l, int r) { return (r & 3) + 4 * (l >> 5) + 8 * (r >> 2); }
-    __device__ static inline int col(int l) { return l & 31; }
-    // A (TILE x KSTEP): lane l holds A[l % 32][l / 32]; B (KSTEP x TILE): B[l / 32][l % 32]
-    __device__ static inline int ab_mn(int l) { return l & 31; }
-    __device__ static inline int ab_k(int l) { return l >> 5; }
-};
 
 template <>
 struct Mfma<double> {
@@ -190,7 +173,7 @@ struct MfmaLds {
     size_t ls_off, us_off, ld_off, prow_off, piv_off, bytes;
     __host__ __device__ MfmaLds(int k, bool lg = false)
     {
-        constexpr int TILE = sizeof(T) == 4 ? 32 : 16;
+        constexpr int TILE = 16;
         kp = ((k + TILE - 1) / TILE) * TILE;
         ls_stride = MNB + 1;
         us_stride = kp + 4;
@@ -203,10 +186,10 @@ struct MfmaLds {
     }
 };
 
-// NT threads (256 or 512), one panel row and one U-block column each, so
-// k + 32 <= NT.  LG: -L_below read from the band in the trailing update
-// (MfmaLds lg).
-template <class T, int NT, bool LG>
+// NT threads, one panel row and one U-block column each, so k + 32 <= NT.
+// LG: -L_below read from the band in the trailing update (MfmaLds lg).
+constexpr int NT = 512;
+template <class T, bool LG>
 __global__ __launch_bounds__(NT) void band_factor_mfma_kernel(T* __restrict__ B0, T* __restrict__ B1, int k_all,
                                                                const FactorJob* __restrict__ jobs)
 {
@@ -340,13 +323,12 @@ __global__ __launch_bounds__(NT) void band_factor_mfma_kernel(T* __restrict__ B0
         __syncthreads();
 
         // (4) trailing window -= L_below * U_right on the matrix cores, TG
-        //     tiles per wavefront at a time (8 KB of FP64 or FP32 window): the
-        //     window (and, LG, the
+        //     tiles per wavefront at a time (8 KB of window): the window (and, LG, the
         //     -L_below) loads of the group are issued before its products, so
         //     their latencies overlap; each tile's products run in the same
         //     order as one tile at a time.
         const int nt = (Mw + TILE - 1) / TILE;
-        constexpr int TG = sizeof(T) == 4 ? 2 : 4, NK = MNB / MF::KSTEP;   // 32 x 32 FP32 tiles: two
+        constexpr int TG = 4, NK = MNB / MF::KSTEP;
         for (int e0 = wave; e0 < nt * nt; e0 += NW * TG) {
             typename MF::acc_t acc[TG];
             T av[LG ? TG : 1][NK];
@@ -1205,25 +1187,29 @@ constexpr size_t LDS_LIMIT = 160 * 1024 - 1024;   // leave room for static LDS
 
 }  // namespace
 
-template <class T, int NT, bool LG>
+template <class T, bool LG>
 void launch_factor_mfma(T* B0, T* B1, int k, const FactorJob* jobs, int njobs, hipStream_t st)
 {
     const size_t lds = MfmaLds<T>(k, LG).bytes;
-    SAP_HIP_CHECK(hipFuncSetAttribute((const void*)band_factor_mfma_kernel<T, NT, LG>,
+    SAP_HIP_CHECK(hipFuncSetAttribute((const void*)band_factor_mfma_kernel<T, LG>,
                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    hipLaunchKernelGGL((band_factor_mfma_kernel<T, NT, LG>), dim3(njobs), dim3(NT), lds, st, B0, B1, k, jobs);
+    hipLaunchKernelGGL((band_factor_mfma_kernel<T, LG>), dim3(njobs), dim3(NT), lds, st, B0, B1, k, jobs);
     SAP_LAUNCH_CHECK();
 }
 
-// The matrix-core blocked kernel's variant for half-bandwidth k: 100 (256
-// threads, -L_below in LDS), 101 (512 threads), 102 (512 threads, -L_below
-// from the band); -1 when none applies.
+// The matrix-core blocked kernel for half-bandwidth k: 100 (panel rows and
+// columns by lanes), in FP64 past that 101 (512 threads, -L_below in LDS) and
+// 102 (512 threads, -L_below from the band); -1 when none applies.
+// 100 wherever its panel fits the LDS and the threads: FP64, n = 100000, 16
+// partitions: 6.7 ms at k = 224 against 15.5 by a row per thread.
 template <class T>
 int factor_mfma_variant(int k)
 {
-    if (k + MNB <= 256 && MfmaLds<T>(k).bytes <= LDS_LIMIT) return 100;
-    if (k + MNB <= 512 && MfmaLds<T>(k).bytes <= LDS_LIMIT) return 101;
-    if (k + MNB <= 512 && MfmaLds<T>(k, true).bytes <= LDS_LIMIT) return 102;
+    if (band_factor_window_fits<T>(k)) return 100;
+    if constexpr (sizeof(T) == 8) {
+        if (k + MNB <= NT && MfmaLds<T>(k).bytes <= LDS_LIMIT) return 101;
+        if (k + MNB <= NT && MfmaLds<T>(k, true).bytes <= LDS_LIMIT) return 102;
+    }
     return -1;
 }
 
@@ -1246,11 +1232,11 @@ void launch_band_factor(T* B0, T* B1, const T* Bin, int k, const FactorJob* d_jo
     if (njobs <= 0) return;
     if (launch_band_factor_resident<T>(B0, B1, Bin, k, d_jobs, njobs, max_len, st)) return;
     if (Bin) throw Error(SAP_ERR_HIP, "separate-input factorization needs the register-resident kernel");
-    switch (factor_mfma_variant<T>(k)) {
-    case 100: launch_factor_mfma<T, 256, false>(B0, B1, k, d_jobs, njobs, st); return;
-    case 101: launch_factor_mfma<T, 512, false>(B0, B1, k, d_jobs, njobs, st); return;
-    case 102: launch_factor_mfma<T, 512, true>(B0, B1, k, d_jobs, njobs, st); return;
-    default: break;
+    if (launch_band_factor_window<T>(B0, B1, k, d_jobs, njobs, st)) return;
+    if constexpr (sizeof(T) == 8) {
+        const int mv = factor_mfma_variant<T>(k);
+        if (mv == 101) { launch_factor_mfma<T, false>(B0, B1, k, d_jobs, njobs, st); return; }
+        if (mv == 102) { launch_factor_mfma<T, true>(B0, B1, k, d_jobs, njobs, st); return; }
     }
     if (factor_lds_bytes<T>(k, 32) <= LDS_LIMIT)      launch_factor_nb<T, 32>(B0, B1, k, d_jobs, njobs, st);
     else if (factor_lds_bytes<T>(k, 16) <= LDS_LIMIT) launch_factor_nb<T, 16>(B0, B1, k, d_jobs, njobs, st);

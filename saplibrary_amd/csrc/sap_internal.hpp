@@ -248,6 +248,12 @@ bool band_factor_resident_fits(int k, int64_t max_len);
 template <class T>
 bool launch_band_factor_resident(T* B0, T* B1, const T* Bin, int k, const FactorJob* d_jobs, int njobs,
                                  int64_t max_len, hipStream_t st);
+// Blocked factorization with the window in global memory (wider bands, and
+// partitions of any size)
+template <class T>
+bool band_factor_window_fits(int k);
+template <class T>
+bool launch_band_factor_window(T* B0, T* B1, int k, const FactorJob* d_jobs, int njobs, hipStream_t st);
 // Which factorization kernel launch_band_factor uses for half-bandwidth k
 // (jobs of one launch with their own widths, FactorJob::kb, must share it;
 // the launch then takes the largest of their widths as its k).
