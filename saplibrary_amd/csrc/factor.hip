@@ -1308,34 +1308,39 @@ void launch_reduced_factor(const T* WV, int k, int nb, T* S, T* Sinv, int safe, 
     const unsigned tiles = (unsigned)((k + GT - 1) / GT);
     hipLaunchKernelGGL(schur_gemm_kernel<T>, dim3(nb, tiles, tiles), dim3(256), 0, st, WV, k, S);
     SAP_LAUNCH_CHECK();
+    // LU of S_i in registers up to k = 224 (FP32) / 160 (FP64), in LDS while it
+    // fits, else in global memory; the inverse by the blocked matrix-core
+    // sweeps wherever those fit.  (FP64, k = 150, 31 boundaries, whose matrix is
+    // too large for the LDS: 0.21 and 0.07 ms, against 1.24 and 0.47 ms in
+    // global memory and column by column.)
     const size_t lds_lu = sizeof(T) * (size_t)k * k;
-    if (lds_lu <= LDS_LIMIT && k <= 256) {
-        // LU in LDS; the inverse by the blocked matrix-core sweeps when they fit
-        const bool mfma_inv = k <= 32 * STK_IT && StkLayout<T>(k).bytes() <= LDS_LIMIT;
-        if (!mfma_inv || !launch_schur_lu_reg<T, 1>(S, k, nb, safe, st)) {
+    const bool mfma_inv = k <= 32 * STK_IT && StkLayout<T>(k).bytes() <= LDS_LIMIT;
+    if (!mfma_inv || !launch_schur_lu_reg<T, 1>(S, k, nb, safe, st)) {
+        if (lds_lu <= LDS_LIMIT && k <= 256) {
             SAP_HIP_CHECK(hipFuncSetAttribute((const void*)schur_lu_inv_kernel<T>,
                                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_lu));
             hipLaunchKernelGGL(schur_lu_inv_kernel<T>, dim3(nb), dim3(1024), lds_lu, st, S, Sinv, k, safe,
                                mfma_inv ? 0 : 1);
             SAP_LAUNCH_CHECK();
-        }
-        if (mfma_inv) {
-            const size_t lds = StkLayout<T>(k).bytes();
-            constexpr int NR = StkCfg<T>::NR;
-            SAP_HIP_CHECK(hipFuncSetAttribute((const void*)schur_inverse_mfma_kernel<T>,
-                                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-            hipLaunchKernelGGL(schur_inverse_mfma_kernel<T>, dim3(nb, (k + NR - 1) / NR), dim3(STK_THREADS), lds, st,
-                               S, k, Sinv);
+            if (!mfma_inv) return;
+        } else {
+            hipLaunchKernelGGL(schur_lu_kernel<T>, dim3(nb), dim3(256), 0, st, S, k, safe);
             SAP_LAUNCH_CHECK();
         }
-        return;
     }
-    hipLaunchKernelGGL(schur_lu_kernel<T>, dim3(nb), dim3(256), 0, st, S, k, safe);
-    SAP_LAUNCH_CHECK();
-    const size_t lds = sizeof(T) * (size_t)k * (RC + 1);
-    SAP_HIP_CHECK(hipFuncSetAttribute((const void*)schur_inverse_kernel<T>,
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    hipLaunchKernelGGL(schur_inverse_kernel<T>, dim3(nb, (k + RC - 1) / RC), dim3(256), lds, st, S, k, Sinv);
+    if (mfma_inv) {
+        const size_t lds = StkLayout<T>(k).bytes();
+        constexpr int NR = StkCfg<T>::NR;
+        SAP_HIP_CHECK(hipFuncSetAttribute((const void*)schur_inverse_mfma_kernel<T>,
+                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        hipLaunchKernelGGL(schur_inverse_mfma_kernel<T>, dim3(nb, (k + NR - 1) / NR), dim3(STK_THREADS), lds, st, S,
+                           k, Sinv);
+    } else {
+        const size_t lds = sizeof(T) * (size_t)k * (RC + 1);
+        SAP_HIP_CHECK(hipFuncSetAttribute((const void*)schur_inverse_kernel<T>,
+                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        hipLaunchKernelGGL(schur_inverse_kernel<T>, dim3(nb, (k + RC - 1) / RC), dim3(256), lds, st, S, k, Sinv);
+    }
     SAP_LAUNCH_CHECK();
 }
 
