@@ -1,0 +1,43 @@
+// Allocation of the library's device buffers.
+#include "sap_internal.hpp"
+
+#include <atomic>
+#include <cstdlib>
+
+namespace sap_amd {
+
+namespace {
+
+std::atomic<size_t> g_held{0};   // bytes of all buffers
+
+// SAP_AMD_DEVICE_LIMIT, 0 when unset
+size_t held_limit()
+{
+    const char* e = std::getenv("SAP_AMD_DEVICE_LIMIT");
+    return e ? (size_t)std::strtoull(e, nullptr, 10) : 0;
+}
+
+}  // namespace
+
+void* device_alloc(size_t bytes)
+{
+    const size_t limit = held_limit();
+    void* p = nullptr;
+    const hipError_t e = hipMalloc(&p, limit && g_held + bytes > limit ? (size_t)1 << 48 : bytes);
+    if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();
+        throw Error(SAP_ERR_OOM, "device buffer of " + std::to_string(bytes) + " bytes beside " +
+                                     std::to_string(g_held) + " held: " + hipGetErrorString(e));
+    }
+    SAP_HIP_CHECK(e);
+    g_held += bytes;
+    return p;
+}
+
+void device_free(void* p, size_t bytes)
+{
+    (void)hipFree(p);
+    g_held -= bytes;
+}
+
+}  // namespace sap_amd

@@ -190,11 +190,12 @@ namespace {
 
 // Out-of-memory for the SaP-C buffers can be forced from the host
 // (SAP_AMD_FAIL_SPIKE_ALLOC=1 in the environment), so the fallback below
-// is testable without exhausting the device.
-bool spike_alloc_forced_to_fail()
+// is testable without exhausting the device: an allocation of more than any
+// device has.
+void fail_spike_alloc_if_asked()
 {
     const char* e = std::getenv("SAP_AMD_FAIL_SPIKE_ALLOC");
-    return e && e[0] == '1';
+    if (e && e[0] == '1') DevBuf<char>((size_t)1 << 48);
 }
 
 int clamp_partitions(int64_t n, int k, int requested)
@@ -216,7 +217,7 @@ bool Precond<T>::try_spike_buffers(A alloc, R release)
 {
     if (block_fallback_) return false;
     try {
-        if (spike_alloc_forced_to_fail()) throw Error(SAP_ERR_OOM, "SaP-C buffers (forced)");
+        fail_spike_alloc_if_asked();
         alloc();
         return true;
     } catch (const Error& e) {

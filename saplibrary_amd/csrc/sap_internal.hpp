@@ -19,16 +19,28 @@ struct Error : public std::runtime_error {
     Error(int c, const std::string& m) : std::runtime_error(m), code(c) {}
 };
 
+// (the failure is taken out of the thread's last error too: the runtime keeps
+// it there over later successful calls, and the next launch check would report
+// it again, for instance after a caught SAP_ERR_OOM)
 #define SAP_HIP_CHECK(expr)                                                              \
     do {                                                                                 \
         hipError_t _e = (expr);                                                          \
         if (_e != hipSuccess) {                                                          \
+            (void)hipGetLastError();                                                     \
             throw ::sap_amd::Error(_e == hipErrorOutOfMemory ? SAP_ERR_OOM : SAP_ERR_HIP, \
                                    std::string(#expr) + ": " + hipGetErrorString(_e));    \
         }                                                                                \
     } while (0)
 
 #define SAP_LAUNCH_CHECK() SAP_HIP_CHECK(hipGetLastError())
+
+// Device memory of the library's buffers (memory.hip).  An allocation that does
+// not fit throws SAP_ERR_OOM.  SAP_AMD_DEVICE_LIMIT=<bytes> in the environment
+// bounds what the buffers may hold together, so that the paths for a full
+// device are testable on an empty one: past the limit the request is made for
+// more than any device has, and fails as the device's own memory would.
+void* device_alloc(size_t bytes);
+void device_free(void* p, size_t bytes);
 
 // Owning device allocation.
 template <class T>
@@ -49,12 +61,12 @@ public:
     {
         if (n == n_) return;
         release();
-        if (n) SAP_HIP_CHECK(hipMalloc(&p_, n * sizeof(T)));
+        if (n) p_ = static_cast<T*>(device_alloc(n * sizeof(T)));
         n_ = n;
     }
     void release()
     {
-        if (p_) (void)hipFree(p_);
+        if (p_) device_free(p_, n_ * sizeof(T));
         p_ = nullptr;
         n_ = 0;
     }
