@@ -92,7 +92,7 @@ void Precond<T>::factor(const std::vector<FactorJob>& jobs)
 template <class T>
 void Precond<T>::begin_tables(int ranges, int kmax, bool with_ul)
 {
-    tabs_on_ = sweep_max_nbuf<T>(kmax) > 0;
+    tabs_on_ = !tabs_denied_ && sweep_max_nbuf<T>(kmax) > 0;
     if (!tabs_on_) {
         tab_[0].release();
         tab_[1].release();
@@ -109,6 +109,22 @@ void Precond<T>::begin_tables(int ranges, int kmax, bool with_ul)
         tab_[1].release();
         tabs_on_ = false;
     }
+}
+
+template <class T>
+bool Precond<T>::drop_tables()
+{
+    if (!tab_[0].size() && !tab_[1].size()) return false;
+    // (a sweep may still read them)
+    SAP_HIP_CHECK(hipStreamSynchronize(stream));
+    if (side_.s) SAP_HIP_CHECK(hipStreamSynchronize(side_.s));
+    if (side2_.s) SAP_HIP_CHECK(hipStreamSynchronize(side2_.s));
+    tab_[0].release();
+    tab_[1].release();
+    tabs_on_ = false;
+    for (VJobs& J : vjobs_) J.n = 0;      // the job tables name them
+    for (BcrJobs& J : bjobs_) J.nr = 0;
+    return true;
 }
 
 template <class T>
@@ -216,12 +232,15 @@ template <class A, class R>
 bool Precond<T>::try_spike_buffers(A alloc, R release)
 {
     if (block_fallback_) return false;
-    try {
-        fail_spike_alloc_if_asked();
-        alloc();
-        return true;
-    } catch (const Error& e) {
-        if (e.code != SAP_ERR_OOM) throw;
+    for (;;) {
+        try {
+            fail_spike_alloc_if_asked();
+            alloc();
+            return true;
+        } catch (const Error& e) {
+            if (e.code != SAP_ERR_OOM) throw;
+        }
+        if (drop_tables()) continue;   // (the last setup's)
         release();
         block_fallback_ = true;
         return false;
@@ -294,6 +313,12 @@ void Precond<T>::begin_setup(int64_t n_, int k_, bool const_band)
 
 template <class T>
 int Precond<T>::setup(int64_t n_, int k_, const double* d_band)
+{
+    return with_room([&] { return setup_steps(n_, k_, d_band); });
+}
+
+template <class T>
+int Precond<T>::setup_steps(int64_t n_, int k_, const double* d_band)
 {
     reorder_ = scale_ = var_mode_ = false;
     row_perm_.release(); col_reord_.release(); row_scale_.release(); col_scale_.release();
@@ -379,6 +404,13 @@ void Precond<T>::tune_sweeps()
 template <class T>
 int Precond<T>::setup_csr(int64_t n_, int64_t nnz, const int* d_rp, const int* d_ci, const double* d_val,
                           const ReorderConfig& rc)
+{
+    return with_room([&] { return setup_csr_steps(n_, nnz, d_rp, d_ci, d_val, rc); });
+}
+
+template <class T>
+int Precond<T>::setup_csr_steps(int64_t n_, int64_t nnz, const int* d_rp, const int* d_ci, const double* d_val,
+                                const ReorderConfig& rc)
 {
     Events ev;
     var_mode_ = false;
@@ -643,6 +675,13 @@ bool Precond<T>::update(const double* d_entries, int64_t count, int* rc)
         throw Error(SAP_ERR_ILLEGAL_UPDATE, "Illegal call to update() with reordering tracking disabled.");
     if (count != src_count_) return false;
     if (cfg.precondType == SAP_None) return true;
+    *rc = with_room([&] { return update_steps(d_entries, count); });
+    return true;
+}
+
+template <class T>
+int Precond<T>::update_steps(const double* d_entries, int64_t count)
+{
     finish_pending();
     const double t0 = std::chrono::duration<double, std::milli>(
         std::chrono::steady_clock::now().time_since_epoch()).count();
@@ -667,8 +706,7 @@ bool Precond<T>::update(const double* d_entries, int64_t count, int* rc)
     tm_.span(&time_toBanded, 0, 1);
     time_cpu_assemble = std::chrono::duration<double, std::milli>(
         std::chrono::steady_clock::now().time_since_epoch()).count() - t0;
-    *rc = factor_band();
-    return true;
+    return factor_band();
 }
 
 template <class T>
@@ -755,6 +793,23 @@ int Precond<T>::var_factor_steps()
     split_ = false;
     vjobs_[0].n = vjobs_[1].n = 0;   // the sweep job tables are built again for these bands
     offB_.release(); offC_.release(); Bul_.release(); scr1_.release();
+    // (before the sweeps' tables, which the setup can do without)
+    const size_t kk = (size_t)k * k;
+    if (spike_active())
+        (void)try_spike_buffers(
+            [&] {
+                g_.resize(n);
+                gd_.resize(n);
+                vq_.resize(n);
+                WV_.resize(2 * kk * (P - 1));
+                S_.resize(kk * (P - 1));
+                Sinv_.resize(kk * (P - 1));
+                corr_.resize((size_t)2 * k * (P - 1));
+            },
+            [&] {
+                WV_.release(); S_.release(); Sinv_.release(); corr_.release(); g_.release(); gd_.release();
+                vq_.release();
+            });
     // one launch per factorization kernel; the jobs of a launch keep their
     // own widths (FactorJob::kb) and band offsets
     std::vector<std::pair<int, int>> order;   // (kernel class, partition)
@@ -809,22 +864,6 @@ int Precond<T>::var_factor_steps()
     tm_.span(&time_bandLU, 3, 4);
     actual_nnz = vboff_[P] - count_band_zeros<T>(Bv_.get(), vboff_[P], (const T*)nullptr, 0, cnt_.get(), stream);
 
-    const size_t kk = (size_t)k * k;
-    if (spike_active())
-        (void)try_spike_buffers(
-            [&] {
-                g_.resize(n);
-                gd_.resize(n);
-                vq_.resize(n);
-                WV_.resize(2 * kk * (P - 1));
-                S_.resize(kk * (P - 1));
-                Sinv_.resize(kk * (P - 1));
-                corr_.resize((size_t)2 * k * (P - 1));
-            },
-            [&] {
-                WV_.release(); S_.release(); Sinv_.release(); corr_.release(); g_.release(); gd_.release();
-                vq_.release();
-            });
     if (!spike_active()) {
         WV_.release(); S_.release(); Sinv_.release(); corr_.release(); g_.release(); gd_.release(); vq_.release();
         return 0;
@@ -1312,6 +1351,12 @@ void Precond<T>::solve_band(const double* v, double* z)
 
 template <class T>
 void Precond<T>::reserve_multi(int nr)
+{
+    with_room([&] { reserve_multi_steps(nr); });
+}
+
+template <class T>
+void Precond<T>::reserve_multi_steps(int nr)
 {
     // (a batched solve may capture apply_multi into a graph: the main stream
     // is ordered after the deferred setup work here, outside the capture)

@@ -153,6 +153,26 @@ public:
     // Allocates apply_multi's work buffers for nr columns (so that a later
     // apply_multi, e.g. under graph capture, allocates nothing).
     void reserve_multi(int nr);
+    // Releases the sweeps' tables (the sweeps are then the plain blocked ones,
+    // until the next setup or update); false when there are none.
+    bool drop_tables();
+    // make(), an allocation (or a whole setup) that can be repeated: once more
+    // without the tables, which only save time, when the device is full
+    template <class F>
+    auto with_room(F make) -> decltype(make())
+    {
+        try {
+            return make();
+        } catch (const Error& e) {
+            if (e.code != SAP_ERR_OOM || !drop_tables()) throw;
+        }
+        struct Denied {
+            bool& d;
+            explicit Denied(bool& d_) : d(d_) { d = true; }
+            ~Denied() { d = false; }
+        } denied(tabs_denied_);
+        return make();
+    }
     // Appends the full-sweep jobs of this preconditioner for nr columns
     // (input at voff + r*n, output at ooff + r*n, gates gate0 + r) to a
     // launch that covers several systems; false (nothing appended) unless
@@ -206,6 +226,12 @@ private:
     DevBuf<T> tab_[2];
     int64_t tab_stride_ = 0;
     bool tabs_on_ = false;
+    bool tabs_denied_ = false;   // a setup repeated without them (with_room)
+    int setup_steps(int64_t n_, int k_, const double* d_band);
+    int setup_csr_steps(int64_t n_, int64_t nnz, const int* d_rp, const int* d_ci, const double* d_val,
+                        const ReorderConfig& rc);
+    int update_steps(const double* d_entries, int64_t count);
+    void reserve_multi_steps(int nr);
     // sizes the tables for `ranges` factored ranges over the n rows
     void begin_tables(int ranges, int kmax, bool with_ul);
     void make_tables(const T* b0, const T* b1, int kl, size_t first, int njobs, int64_t max_len);

@@ -264,6 +264,14 @@ public:
         else if (pd) fin(*pd);
     }
 
+    bool drop_tables() { return pf ? pf->drop_tables() : pd->drop_tables(); }
+    template <class F>
+    void with_room(F make)
+    {
+        if (pf) pf->with_room(make);
+        else pd->with_room(make);
+    }
+
     // ---------------------------------------------------------- vectors
     void reserve_vectors(int count)
     {
@@ -273,8 +281,10 @@ public:
             if (ext_work_size_ < need) throw Error(SAP_ERR_BADARG, "solve work space too small");
             base = ext_work_;
         } else {
-            if (work_.size() < need) work_.resize(need);
-            partials_.resize(dot_partials_size());
+            with_room([&] {
+                if (work_.size() < need) work_.resize(need);
+                partials_.resize(dot_partials_size());
+            });
             base = work_.get();
         }
         vecs_.clear();
@@ -877,7 +887,7 @@ public:
             std::vector<int64_t> off(nr);
             std::vector<int> len(nr, (int)n);
             for (int c = 0; c < nr; ++c) off[c] = (int64_t)c * n;
-            batch_ = std::make_unique<BatchKrylov>(stream, off, len);
+            with_room([&] { batch_ = std::make_unique<BatchKrylov>(stream, off, len); });
             batch_n_ = n;
         }
         // the preconditioner's work buffers exist before any graph capture
@@ -1056,11 +1066,28 @@ public:
     {
         const double t0 = wall_ms();
         for (size_t s = 0; s < sys.size(); ++s) {
-            const int rc = sys[s]->setup_banded(n[s], k[s], bands[s]);
+            int rc = 0;
+            with_room([&] { rc = sys[s]->setup_banded(n[s], k[s], bands[s]); });
             if (rc != 0) return rc;
         }
         timeSetup = wall_ms() - t0;
         return 0;
+    }
+    // make(), an allocation or a setup that can be repeated: once more without
+    // any system's sweep tables when the device is full
+    template <class F>
+    void with_room(F make)
+    {
+        try {
+            make();
+            return;
+        } catch (const Error& e) {
+            bool any = false;
+            if (e.code == SAP_ERR_OOM)
+                for (auto& p : sys) any = p->drop_tables() || any;
+            if (!any) throw;
+        }
+        make();
     }
 
     struct Ops : BatchOps {
@@ -1134,15 +1161,19 @@ public:
                     at += n_[s];
                 }
             }
-            kry_ = std::make_unique<BatchKrylov>(stream, off, len);
-            Bb_.resize(at);
-            Xb_.resize(at);
+            with_room([&] {
+                kry_ = std::make_unique<BatchKrylov>(stream, off, len);
+                Bb_.resize(at);
+                Xb_.resize(at);
+            });
         }
-        for (int s = 0; s < S; ++s) {
-            Solver& q = *sys[s];
-            if (q.pf) q.pf->reserve_multi(nr_[s]);
-            else q.pd->reserve_multi(nr_[s]);
-        }
+        with_room([&] {
+            for (int s = 0; s < S; ++s) {
+                Solver& q = *sys[s];
+                if (q.pf) q.pf->reserve_multi(nr_[s]);
+                else q.pd->reserve_multi(nr_[s]);
+            }
+        });
         // one sweep launch for all systems when every system's apply is a
         // single full sweep pass (the job table depends on the setup's
         // buffers, so it is built for every solve)

@@ -5,6 +5,8 @@ runtime as the device's own memory would.
   * The sweeps' tables are optional (they only make the sweeps faster): a
     setup without room for them succeeds, with the plain sweeps, and gives the
     same preconditioner.
+  * They give way to what cannot be done without: the SaP-C buffers and work
+    space of the same setup, a solve's vectors, the next setup's larger band.
 
 Tolerances: both sweep variants carry the operator's own rounding, as in the
 staged sweeps' and the application tests: 1e-13 (block-diagonal) and 1e-10
@@ -83,3 +85,115 @@ def test_without_room_for_the_tables(sap, oracle, limit, kind, prec_double):
     tol = 3e-5 if not prec_double else 1e-13 if kind == "block" else 1e-10
     for got in (z, zt):
         np.testing.assert_allclose(got, ref, rtol=0, atol=tol * np.abs(ref).max())
+
+
+# The tables of n rows (one band, FP32): both directions of 264 bytes a row and
+# one padded block per partition.
+def tables_bytes(n, P):
+    return 2 * (n // 32 + P) * 8448
+
+
+def spike_options(sap, **kw):
+    return sap.Options(precondType=sap.Spike, factMethod=sap.LU_only, trackReordering=1, relTol=1e-10, refine=8, **kw)
+
+
+# LU_only: the spike tips' work space (n x 32 values) is needed after the tables
+def test_tables_give_way_to_the_setup(sap, oracle, limit):
+    n, k, P = 60000, 20, 8
+    band, v = oracle.gen_banded(n, k, 1.2, 83), torch.from_numpy(oracle.gen_vector(n, 84)).cuda()
+    A = sap.BandedMatrix(torch.from_numpy(band).cuda())
+    cpu = oracle.Solver(P, fact="LU_only", precond="Spike", prec_double=False)
+    assert cpu.setup(band) == 0
+    ref = cpu.apply(v.cpu().numpy())
+    limit((2 * k + 1) * 4 * n + tables_bytes(n, P) + 40 * n)
+    g = sap.Solver(P, spike_options(sap))
+    g.setup(A)
+    np.testing.assert_allclose(apply(g, v), ref, rtol=0, atol=3e-5 * np.abs(ref).max())
+    g.update(A.band)
+    np.testing.assert_allclose(apply(g, v), ref, rtol=0, atol=3e-5 * np.abs(ref).max())
+
+
+def test_tables_give_way_to_the_solve_and_the_next_setup(sap, oracle, limit):
+    n, k, P = 60000, 20, 8
+    A = sap.BandedMatrix(torch.from_numpy(oracle.gen_banded(n, k, 1.2, 85)).cuda())
+    big = sap.BandedMatrix(torch.from_numpy(oracle.gen_banded(3 * n // 2, k, 1.2, 86)).cuda())
+    # the band, its vectors and the tables; a solve takes 32 FP64 vectors more
+    limit((2 * k + 1) * 4 * n + tables_bytes(n, P) + 40 * n)
+    g = sap.Solver(P, sap.Options(precondType=sap.Block, relTol=1e-10, refine=8))
+    g.setup(A)
+    for M in (A, big):
+        if M is big:
+            limit((2 * k + 1) * 4 * M.num_rows + (40 + 256) * M.num_rows + MIB)
+            g.setup(M)
+        x0 = torch.rand(M.num_rows, dtype=torch.float64, device="cuda")
+        b = sap.band_spmv(M, x0, torch.empty_like(x0))
+        x = torch.zeros_like(b)
+        assert g.solve(None, b, x), g.getMonitorMessage()
+        r = b - sap.band_spmv(M, x, torch.empty_like(x))
+        assert float(r.norm() / b.norm()) <= 1e-10
+
+
+def test_tables_give_way_to_a_batch(sap, oracle, limit):
+    n, k, P, nr = 30000, 20, 8, 1
+    mats = [sap.BandedMatrix(torch.from_numpy(oracle.gen_banded(n, k, 1.2, 87 + s)).cuda()) for s in range(3)]
+    B = [torch.rand(n, nr, dtype=torch.float64, device="cuda") for _ in mats]
+
+    def run():
+        b = sap.SystemBatch([P] * len(mats), sap.Options(precondType=sap.Block, relTol=1e-10, refine=8))
+        b.setup(mats)
+        X = [torch.zeros_like(c) for c in B]
+        assert b.solve(B, X)
+        return X
+    ref = run()
+    gc.collect()
+    one = (2 * k + 1) * 4 * n + 40 * n + tables_bytes(n, P)
+    for cap in (2 * one + one // 2,                              # the third system's tables do not fit
+                3 * one + MIB,                                   # the solve's vectors do not
+                3 * (one - tables_bytes(n, P)) + 3 * n * 8 * 24):  # nor does the third system
+        limit(cap)
+        try:
+            X = run()
+        finally:
+            limit(None)
+        gc.collect()
+        for x, y in zip(X, ref):
+            assert float((x - y).norm() / y.norm()) <= 1e-9
+
+
+# Variable bandwidth: with less and less memory the setup is truncated SPIKE with
+# the tables, then without, and only then anything else.
+def test_tables_give_way_to_the_spike_buffers(sap, oracle, limit):
+    from tests.csr_cases import sparse_band
+    n, P = 6000, 3
+    rp, ci, val = sparse_band(n, 90, 8, 57)
+    A = sap.CsrMatrix.from_host(rp, ci, val)
+    v = torch.from_numpy(oracle.gen_vector(n, 404)).cuda()
+    opts = sap.Options(precValueType=sap.PREC_DOUBLE)
+    g = sap.Solver(P, opts)
+    g.setup(A)
+    full = apply(g, v)
+    tol = 1e-10 * np.abs(full).max()
+    del g
+    gc.collect()
+    seen = []
+    for cap in range(32 * MIB, 0, -MIB // 4):
+        limit(cap)
+        g = None
+        try:
+            g = sap.Solver(P, opts)
+            g.setup(A)
+            z = apply(g, v)
+            seen.append("tables" if np.array_equal(z, full) else "spike" if np.abs(z - full).max() <= tol else "other")
+        except sap.SapError as e:
+            assert "Out_of_memory" in str(e) or g is None, str(e)
+            seen.append("oom")
+        finally:
+            limit(None)
+            del g
+            gc.collect()
+        if seen[-1] == "oom" and len(seen) > 4 and seen[-4:] == ["oom"] * 4:
+            break
+    print("[memory] " + " ".join(seen), flush=True)
+    order = ["tables", "spike"]
+    good = [s for s in seen if s in order]
+    assert seen[:len(good)] == sorted(good, key=order.index) and "tables" in good and "spike" in good
