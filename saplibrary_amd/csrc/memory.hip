@@ -10,10 +10,10 @@ namespace {
 
 std::atomic<size_t> g_held{0};   // bytes of all buffers
 
-// SAP_AMD_DEVICE_LIMIT, 0 when unset
-size_t held_limit()
+// a number of bytes in the environment, 0 when unset
+size_t env_bytes(const char* name)
 {
-    const char* e = std::getenv("SAP_AMD_DEVICE_LIMIT");
+    const char* e = std::getenv(name);
     return e ? (size_t)std::strtoull(e, nullptr, 10) : 0;
 }
 
@@ -21,7 +21,7 @@ size_t held_limit()
 
 void* device_alloc(size_t bytes)
 {
-    const size_t limit = held_limit();
+    const size_t limit = env_bytes("SAP_AMD_DEVICE_LIMIT");
     void* p = nullptr;
     const hipError_t e = hipMalloc(&p, limit && g_held + bytes > limit ? (size_t)1 << 48 : bytes);
     if (e == hipErrorOutOfMemory) {
@@ -38,6 +38,14 @@ void device_free(void* p, size_t bytes)
 {
     (void)hipFree(p);
     g_held -= bytes;
+}
+
+size_t device_free_bytes()
+{
+    if (const size_t set = env_bytes("SAP_AMD_DEVICE_FREE")) return set;
+    size_t free = 0, total = 0;
+    SAP_HIP_CHECK(hipMemGetInfo(&free, &total));
+    return free;
 }
 
 }  // namespace sap_amd

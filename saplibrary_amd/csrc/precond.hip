@@ -99,10 +99,25 @@ void Precond<T>::begin_tables(int ranges, int kmax, bool with_ul)
         return;
     }
     tab_stride_ = sweep_tab_elems<T>(n, ranges);
+    const size_t want[2] = {(size_t)(2 * tab_stride_), with_ul ? (size_t)(2 * tab_stride_) : 0};
+    // At most a quarter of the free memory, so that three quarters are left
+    // for what is allocated next, here or by the program: another solver, the
+    // columns of a batch, the program's own arrays.  (For narrow bands the
+    // tables are by far the largest buffer: 528 bytes a row and band in FP32,
+    // against 44 of the band itself at k = 5.)
+    size_t more = 0;
+    for (int i = 0; i < 2; ++i)
+        if (tab_[i].size() != want[i]) {
+            tab_[i].release();
+            more += want[i] * sizeof(T);
+        }
+    if (more && more > device_free_bytes() / 4) {
+        (void)drop_tables();
+        tabs_on_ = false;
+        return;
+    }
     try {
-        tab_[0].resize((size_t)(2 * tab_stride_));
-        if (with_ul) tab_[1].resize((size_t)(2 * tab_stride_));
-        else tab_[1].release();
+        for (int i = 0; i < 2; ++i) tab_[i].resize(want[i]);
     } catch (const Error& e) {
         if (e.code != SAP_ERR_OOM) throw;
         tab_[0].release();

@@ -41,6 +41,8 @@ struct Error : public std::runtime_error {
 // more than any device has, and fails as the device's own memory would.
 void* device_alloc(size_t bytes);
 void device_free(void* p, size_t bytes);
+// device memory that is free now (SAP_AMD_DEVICE_FREE=<bytes>: taken as free)
+size_t device_free_bytes();
 
 // Owning device allocation.
 template <class T>

@@ -7,6 +7,9 @@ runtime as the device's own memory would.
     same preconditioner.
   * They give way to what cannot be done without: the SaP-C buffers and work
     space of the same setup, a solve's vectors, the next setup's larger band.
+  * They take at most a quarter of the memory that is free (what that is taken
+    to be is set with SAP_AMD_DEVICE_FREE), so that what another solver or the
+    program allocates next fits as it does beside a solver without tables.
 
 Tolerances: both sweep variants carry the operator's own rounding, as in the
 staged sweeps' and the application tests: 1e-13 (block-diagonal) and 1e-10
@@ -197,3 +200,25 @@ def test_tables_give_way_to_the_spike_buffers(sap, oracle, limit):
     order = ["tables", "spike"]
     good = [s for s in seen if s in order]
     assert seen[:len(good)] == sorted(good, key=order.index) and "tables" in good and "spike" in good
+
+
+def test_tables_take_a_quarter_of_the_free_memory(sap, oracle, limit, monkeypatch):
+    n, k, P = 60000, 20, 8
+    A = sap.BandedMatrix(torch.from_numpy(oracle.gen_banded(n, k, 1.2, 91)).cuda())
+    v = torch.from_numpy(oracle.gen_vector(n, 92)).cuda()
+    size = 2 * (n // 32 + P) * 2112 * 4   # of the tables: (n / 32 + P) blocks of 2112 values, two directions
+
+    def z_with(free):
+        if free:
+            monkeypatch.setenv("SAP_AMD_DEVICE_FREE", str(free))
+        g = sap.Solver(P, sap.Options(precondType=sap.Block))
+        g.setup(A)
+        monkeypatch.delenv("SAP_AMD_DEVICE_FREE", raising=False)
+        return apply(g, v)
+    full = z_with(0)
+    limit((2 * k + 1) * 4 * n + 40 * n + 20 * MIB)
+    plain = z_with(0)
+    limit(None)
+    assert not np.array_equal(plain, full)
+    assert np.array_equal(z_with(4 * size), full)
+    assert np.array_equal(z_with(4 * size - 4), plain)
