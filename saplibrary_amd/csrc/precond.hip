@@ -90,9 +90,9 @@ void Precond<T>::factor(const std::vector<FactorJob>& jobs)
 }
 
 template <class T>
-void Precond<T>::begin_tables(int ranges, int kmax, bool with_ul)
+void Precond<T>::begin_tables(int ranges, int kmin, bool with_ul)
 {
-    tabs_on_ = !tabs_denied_ && sweep_max_nbuf<T>(kmax) > 0;
+    tabs_on_ = !tabs_denied_ && sweep_max_nbuf<T>(kmin) > 0;
     if (!tabs_on_) {
         tab_[0].release();
         tab_[1].release();
@@ -856,7 +856,7 @@ int Precond<T>::var_factor_steps()
                                      stream));
         jobs_host_ = jobs;
     }
-    begin_tables(P, *std::max_element(vks_.begin(), vks_.end()), false);
+    begin_tables(P, *std::min_element(vks_.begin(), vks_.end()), false);
     tm_.mark(3, stream);
     {
         ProfScope ps(prof, "band_factor");

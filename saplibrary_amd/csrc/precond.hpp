@@ -232,8 +232,10 @@ private:
                         const ReorderConfig& rc);
     int update_steps(const double* d_entries, int64_t count);
     void reserve_multi_steps(int nr);
-    // sizes the tables for `ranges` factored ranges over the n rows
-    void begin_tables(int ranges, int kmax, bool with_ul);
+    // sizes the tables for `ranges` factored ranges over the n rows; kmin: the
+    // narrowest range's half-bandwidth (ranges too wide for the staged sweep
+    // leave their part unused)
+    void begin_tables(int ranges, int kmin, bool with_ul);
     void make_tables(const T* b0, const T* b1, int kl, size_t first, int njobs, int64_t max_len);
     // the tables of range `range` starting at row `start` (LU band)
     SweepTabs<T> range_tabs(int64_t start, int range) const;

@@ -196,6 +196,10 @@ constexpr int SW_THREADS = 768;
 constexpr int SW_DIN = 16;           // right-hand side steps in flight
 constexpr int SW_NIN = SW_DIN + 1;   // staging slots of 64 dwords
 
+// widest band the staged sweep takes (two far rows per lane above 192 + BS)
+template <class T>
+constexpr int sweep_staged_max() { return 2 * SW_FAR + sweep_bs<T>(); }   // (ring B columns: up to 384 far rows)
+
 // Waits until at most n (wave-uniform, 0 .. 63) vector memory operations are
 // outstanding.  s_waitcnt takes an immediate, so this jumps into a table of
 // 64 (wait, branch) pairs of 8 bytes each, which starts 12 bytes after the
@@ -935,6 +939,7 @@ __global__ __launch_bounds__(TAB_THREADS) void sweep_tables_kernel(const T* __re
     __shared__ alignas(16) T lb[NB * BS * LS];   // per block: column m of L in row m; then T, then S
     const FactorJob J = jobs[blockIdx.y];
     const int k = J.kb > 0 ? J.kb : k_all;
+    if (k > sweep_staged_max<T>()) return;   // swept without tables
     const int stage = blockIdx.z;
     const int nblk = (int)((J.len + BS - 1) / BS);
     if ((int)blockIdx.x * NB >= nblk) return;
@@ -1383,10 +1388,6 @@ size_t sweep_lds(int k)
 }
 
 }  // namespace
-
-// widest band the staged sweep takes (two far rows per lane above 192 + BS)
-template <class T>
-constexpr int sweep_staged_max() { return 2 * SW_FAR + sweep_bs<T>(); }   // (ring B columns: up to 384 far rows)
 
 // Sweep configuration: mode and (mode 2) slots of the rings (nbuf as the
 // kernels take it, depth the slots of the deeper one), as many as fit next to

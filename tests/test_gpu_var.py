@@ -259,3 +259,37 @@ def test_var_solve_multi_rhs_and_end_to_end(sap):
     xs = host(xx)
     for c in range(2):
         assert np.linalg.norm(Bm[:, c] - A @ xs[:, c]) / np.linalg.norm(Bm[:, c]) <= 1e-10
+
+
+@pytest.mark.parametrize("prec", ["double", "float"])
+def test_a_wide_partition_leaves_the_others_their_sweeps(sap, monkeypatch, prec):
+    """A 450-row full block at the end of a band of half-width 20: its partition
+    is wider than the staged sweep takes (400 in FP64, 416 in FP32), the others
+    are not and keep it.  So the result has other bits than with the plain
+    sweeps everywhere (no memory for the staged ones' tables), and the same
+    values to rounding."""
+    import scipy.sparse as sp
+    n, P, blk, narrow = 3000, 3, 450, 20
+    r = np.random.default_rng(61)
+    i, j = np.indices((n, n), sparse=True)
+    A = np.where((abs(i - j) <= narrow) | ((i >= n - blk) & (j >= n - blk)), r.uniform(-1, 1, (n, n)), 0.0)
+    np.fill_diagonal(A, 0)
+    np.fill_diagonal(A, 1.5 * np.abs(A).sum(axis=1) + 1)
+    S = sp.csr_matrix(A)
+    S.sort_indices()
+    v = dev(r.uniform(-1, 1, n))
+
+    def run(**kw):
+        g = _setup(sap, S.indptr.astype(np.int32), S.indices.astype(np.int32), S.data, P, prec, **kw)
+        assert g.numPartitions == P and g.getStats().bandwidth > 416
+        out = torch.empty_like(v)
+        g.precond_apply(v, out)
+        return host(out)
+    for kind in (sap.Block, sap.Spike):
+        z = run(precondType=kind)
+        monkeypatch.setenv("SAP_AMD_DEVICE_FREE", "4")
+        plain = run(precondType=kind)
+        monkeypatch.delenv("SAP_AMD_DEVICE_FREE")
+        assert np.isfinite(z).all()
+        np.testing.assert_allclose(z, plain, rtol=0, atol=(1e-12 if prec == "double" else 3e-5) * np.abs(plain).max())
+        assert not np.array_equal(z, plain)
