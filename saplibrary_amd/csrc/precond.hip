@@ -387,7 +387,9 @@ template <class T>
 void Precond<T>::tune_sweeps()
 {
     nbuf_ = 0;
-    if (!cfg.autotune || k == 0 || cfg.precondType == SAP_None) return;
+    // (with variable bandwidth there is no constant-width band to apply, and
+    // the job-table sweeps fix their depth)
+    if (!cfg.autotune || k == 0 || var_mode_ || cfg.precondType == SAP_None) return;
     const int nmax = sweep_max_nbuf<T>(k);
     if (nmax < 4) return;
     std::vector<int> cand;

@@ -293,3 +293,19 @@ def test_a_wide_partition_leaves_the_others_their_sweeps(sap, monkeypatch, prec)
         assert np.isfinite(z).all()
         np.testing.assert_allclose(z, plain, rtol=0, atol=(1e-12 if prec == "double" else 3e-5) * np.abs(plain).max())
         assert not np.array_equal(z, plain)
+
+
+def test_autotune_on_the_variable_path(sap):
+    """options.autotune = 1 with variable bandwidth (no constant-width band
+    exists there to time sweeps on): the same bits as without."""
+    n, P = 2400, 3
+    rp, ci, val = sparse_band(n, 90, 8, 57)
+    v = dev(np.random.default_rng(5).uniform(-1, 1, n))
+    z = []
+    for tune in (0, 1):
+        g = _setup(sap, rp, ci, val, P, "double", autotune=tune)
+        assert g.numPartitions > 1
+        out = torch.empty_like(v)
+        g.precond_apply(v, out)
+        z.append(host(out))
+    assert np.array_equal(z[0], z[1])
