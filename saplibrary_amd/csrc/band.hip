@@ -658,7 +658,7 @@ void launch_band_to_colmajor(int64_t n, int k, const double* band_rm, T* B, hipS
         const int G = 8 * std::max(1, std::min(device_cus() / 8, (int)((nchunks + 7) / 8)));
         const int rpw = (rows + B2C_THREADS / 64 - 1) / (B2C_THREADS / 64);
         auto go = [&](auto kern) {
-            SAP_HIP_CHECK(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+            set_lds_limit((const void*)kern, lds);
             hipLaunchKernelGGL(kern, dim3((unsigned)G), dim3(B2C_THREADS), lds, st, n, k, tc, nchunks, band_rm, B, B2);
         };
         if (rpw <= 8)       go(band_to_colmajor_pipe_kernel<T, 8>);
@@ -666,8 +666,7 @@ void launch_band_to_colmajor(int64_t n, int k, const double* band_rm, T* B, hipS
         else                go(band_to_colmajor_pipe_kernel<T, 32>);
     } else if (tc >= 8) {
         const size_t lds = (size_t)tc * (w + 1) * sizeof(T);
-        SAP_HIP_CHECK(hipFuncSetAttribute((const void*)band_to_colmajor_cols_kernel<T>,
-                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        set_lds_limit((const void*)band_to_colmajor_cols_kernel<T>, lds);
         hipLaunchKernelGGL(band_to_colmajor_cols_kernel<T>, dim3((unsigned)((n + tc - 1) / tc)), dim3(B2C_THREADS),
                            lds, st, n, k, tc, band_rm, B, B2);
     } else {

@@ -1177,8 +1177,7 @@ template <class T, int NB>
 void launch_factor_nb(T* B0, T* B1, int k, const FactorJob* jobs, int njobs, hipStream_t st)
 {
     const size_t lds = factor_lds_bytes<T>(k, NB);
-    SAP_HIP_CHECK(hipFuncSetAttribute((const void*)band_factor_kernel<T, NB>,
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    set_lds_limit((const void*)band_factor_kernel<T, NB>, lds);
     hipLaunchKernelGGL((band_factor_kernel<T, NB>), dim3(njobs), dim3(256), lds, st, B0, B1, k, jobs);
     SAP_LAUNCH_CHECK();
 }
@@ -1191,8 +1190,7 @@ template <class T, bool LG>
 void launch_factor_mfma(T* B0, T* B1, int k, const FactorJob* jobs, int njobs, hipStream_t st)
 {
     const size_t lds = MfmaLds<T>(k, LG).bytes;
-    SAP_HIP_CHECK(hipFuncSetAttribute((const void*)band_factor_mfma_kernel<T, LG>,
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    set_lds_limit((const void*)band_factor_mfma_kernel<T, LG>, lds);
     hipLaunchKernelGGL((band_factor_mfma_kernel<T, LG>), dim3(njobs), dim3(NT), lds, st, B0, B1, k, jobs);
     SAP_LAUNCH_CHECK();
 }
@@ -1270,8 +1268,7 @@ void launch_spike_tips(const T* B, const T* Bul, int k, PartInfo pi, int fact_lu
     if (pi.P < 2) return;
     if (fact_lu_ul && k <= 32 * STK_IT && StkLayout<T>(k).bytes() <= LDS_LIMIT) {
         const size_t lds = StkLayout<T>(k).bytes();
-        SAP_HIP_CHECK(hipFuncSetAttribute((const void*)spike_tips_mfma_kernel<T>,
-                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        set_lds_limit((const void*)spike_tips_mfma_kernel<T>, lds);
         constexpr int NR = StkCfg<T>::NR;
         hipLaunchKernelGGL(spike_tips_mfma_kernel<T>, dim3(pi.P - 1, 2, (k + NR - 1) / NR), dim3(STK_THREADS), lds,
                            st, B, Bul, k, pi, offB, offC, WV);
@@ -1280,8 +1277,7 @@ void launch_spike_tips(const T* B, const T* Bul, int k, PartInfo pi, int fact_lu
     }
     const size_t lds = sizeof(T) * (size_t)k * (RC + 1);
     if (lds > LDS_LIMIT) throw Error(SAP_ERR_UNSUPPORTED, "half-bandwidth too large for the spike kernel");
-    SAP_HIP_CHECK(hipFuncSetAttribute((const void*)spike_tips_kernel<T>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                      (int)lds));
+    set_lds_limit((const void*)spike_tips_kernel<T>, lds);
     const unsigned chunks = (unsigned)((k + RC - 1) / RC);
     if (fact_lu_ul) {
         hipLaunchKernelGGL(spike_tips_kernel<T>, dim3(pi.P - 1, 2, chunks), dim3(256), lds, st, B, Bul, k, pi, offB,
@@ -1317,8 +1313,7 @@ void launch_reduced_factor(const T* WV, int k, int nb, T* S, T* Sinv, int safe, 
     const bool mfma_inv = k <= 32 * STK_IT && StkLayout<T>(k).bytes() <= LDS_LIMIT;
     if (!mfma_inv || !launch_schur_lu_reg<T, 1>(S, k, nb, safe, st)) {
         if (lds_lu <= LDS_LIMIT && k <= 256) {
-            SAP_HIP_CHECK(hipFuncSetAttribute((const void*)schur_lu_inv_kernel<T>,
-                                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_lu));
+            set_lds_limit((const void*)schur_lu_inv_kernel<T>, lds_lu);
             hipLaunchKernelGGL(schur_lu_inv_kernel<T>, dim3(nb), dim3(1024), lds_lu, st, S, Sinv, k, safe,
                                mfma_inv ? 0 : 1);
             SAP_LAUNCH_CHECK();
@@ -1331,14 +1326,12 @@ void launch_reduced_factor(const T* WV, int k, int nb, T* S, T* Sinv, int safe, 
     if (mfma_inv) {
         const size_t lds = StkLayout<T>(k).bytes();
         constexpr int NR = StkCfg<T>::NR;
-        SAP_HIP_CHECK(hipFuncSetAttribute((const void*)schur_inverse_mfma_kernel<T>,
-                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        set_lds_limit((const void*)schur_inverse_mfma_kernel<T>, lds);
         hipLaunchKernelGGL(schur_inverse_mfma_kernel<T>, dim3(nb, (k + NR - 1) / NR), dim3(STK_THREADS), lds, st, S,
                            k, Sinv);
     } else {
         const size_t lds = sizeof(T) * (size_t)k * (RC + 1);
-        SAP_HIP_CHECK(hipFuncSetAttribute((const void*)schur_inverse_kernel<T>,
-                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        set_lds_limit((const void*)schur_inverse_kernel<T>, lds);
         hipLaunchKernelGGL(schur_inverse_kernel<T>, dim3(nb, (k + RC - 1) / RC), dim3(256), lds, st, S, k, Sinv);
     }
     SAP_LAUNCH_CHECK();

@@ -434,8 +434,7 @@ void launch_factor_resident(T* B0, T* B1, const T* Bin, int k, const FactorJob* 
 {
     constexpr int NW = resident_waves<T, KT>();
     const size_t lds = ResLds<T, KT>::bytes;
-    SAP_HIP_CHECK(hipFuncSetAttribute((const void*)band_factor_resident_kernel<T, KT, NW>,
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    set_lds_limit((const void*)band_factor_resident_kernel<T, KT, NW>, lds);
     hipLaunchKernelGGL((band_factor_resident_kernel<T, KT, NW>), dim3(njobs), dim3(64 * NW), lds, st, B0, B1, Bin,
                        k, jobs);
     SAP_LAUNCH_CHECK();

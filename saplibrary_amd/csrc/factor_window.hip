@@ -338,8 +338,7 @@ bool launch_band_factor_window(T* B0, T* B1, int k, const FactorJob* d_jobs, int
 {
     if (!band_factor_window_fits<T>(k)) return false;
     const size_t lds = WinGeom<T>::bytes(k);
-    SAP_HIP_CHECK(hipFuncSetAttribute((const void*)band_factor_window_kernel<T>,
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    set_lds_limit((const void*)band_factor_window_kernel<T>, lds);
     hipLaunchKernelGGL(band_factor_window_kernel<T>, dim3(njobs), dim3(64 * WinGeom<T>::NW), lds, st, B0, B1, k,
                        d_jobs);
     SAP_LAUNCH_CHECK();

@@ -1,8 +1,11 @@
-// Allocation of the library's device buffers.
+// Allocation of the library's device buffers, and the kernels' LDS limits.
 #include "sap_internal.hpp"
 
 #include <atomic>
 #include <cstdlib>
+#include <map>
+#include <mutex>
+#include <utility>
 
 namespace sap_amd {
 
@@ -38,6 +41,19 @@ void device_free(void* p, size_t bytes)
 {
     (void)hipFree(p);
     g_held -= bytes;
+}
+
+void set_lds_limit(const void* kernel, size_t lds)
+{
+    static std::mutex mu;
+    static std::map<std::pair<const void*, int>, size_t> done;
+    int dev = 0;
+    SAP_HIP_CHECK(hipGetDevice(&dev));
+    std::lock_guard<std::mutex> lock(mu);
+    size_t& have = done[{kernel, dev}];
+    if (lds <= have) return;
+    SAP_HIP_CHECK(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    have = lds;
 }
 
 size_t device_free_bytes()

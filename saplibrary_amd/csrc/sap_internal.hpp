@@ -44,6 +44,12 @@ void device_free(void* p, size_t bytes);
 // device memory that is free now (SAP_AMD_DEVICE_FREE=<bytes>: taken as free)
 size_t device_free_bytes();
 
+// Raises a kernel's dynamic LDS limit to lds bytes, once per size and device.
+// Never lowered: launches of the same kernel with other sizes may be under way
+// in other threads.  (Not a stream operation, but a launch whose size has been
+// seen makes no call, so it can be captured into a graph.)
+void set_lds_limit(const void* kernel, size_t lds);
+
 // Owning device allocation.
 template <class T>
 class DevBuf {

@@ -29,9 +29,7 @@
 #include "sap_internal.hpp"
 
 #include <algorithm>
-#include <mutex>
 #include <type_traits>
-#include <unordered_map>
 
 namespace sap_amd {
 
@@ -1418,20 +1416,6 @@ SweepCfg sweep_cfg(int k, bool tabs_ok, int depth_req = 0)
         while (na == nb && na < want && fixed + (na + 1) * (sa + sb) <= LDS_MAX) { ++na; ++nb; }
     }
     return {2, na + 256 * nb, fixed + na * sa + nb * sb, SW_THREADS, nb};
-}
-
-// Raises a kernel's dynamic LDS limit once per size (not a stream
-// operation, but kept out of the launch path so that launches can be
-// captured into a graph with nothing else in between).
-void set_lds_limit(const void* kernel, size_t lds)
-{
-    static std::mutex mu;
-    static std::unordered_map<const void*, size_t> done;
-    std::lock_guard<std::mutex> lock(mu);
-    size_t& have = done[kernel];
-    if (lds <= have) return;
-    SAP_HIP_CHECK(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    have = lds;
 }
 
 template <class T, int MODE>

@@ -106,3 +106,15 @@ def test_cpp_facade_compiles(tmp_path):
     r = subprocess.run([hipcc, "-std=c++17", "-I", os.path.join(ROOT, "include"), "-c", str(src), "-o",
                         str(tmp_path / "facade.o")], capture_output=True, text=True)
     assert r.returncode == 0, r.stderr
+
+
+def test_lds_limits_are_only_raised():
+    """A kernel's dynamic LDS limit is one per process: every launch raises it
+    through set_lds_limit (under a lock, never lowered), so that a launch with
+    a smaller size cannot undercut another thread's."""
+    import glob
+    import os
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    users = [os.path.basename(f) for f in glob.glob(os.path.join(root, "saplibrary_amd", "csrc", "*"))
+             if "hipFuncSetAttribute" in open(f).read()]
+    assert users == ["memory.hip"]

@@ -29,3 +29,37 @@ def test_factors_match_oracle(case, double, fact):
     assert g.numPartitions == cpu.num_partitions
     Fg, Fc = g.factors(), cpu.factors()
     np.testing.assert_allclose(Fg, Fc, rtol=0, atol=(1e-10 if double else 2e-4) * np.abs(Fc).max())
+
+
+def test_two_threads_factor_different_widths():
+    """Setups of two widths at the same time: the kernel's LDS limit, one per
+    process, must never fall below what the other thread's launch needs."""
+    import threading
+    import saplibrary_amd as sap
+    from oracle import pyoracle as oracle
+    opts = dict(factMethod=sap.LU_only, precondType=sap.Block, precValueType=sap.PREC_DOUBLE)
+    bands = [oracle.gen_banded(700, k, 0.8, 26) for k in (113, 224)]
+    one = []
+    for b in bands:
+        g = sap.Solver(1, sap.Options(**opts))
+        g.setup(sap.BandedMatrix(torch.from_numpy(b).cuda()))
+        one.append(g.factors())
+    errors = []
+
+    def work(b, ref):
+        try:
+            st = torch.cuda.Stream()
+            with torch.cuda.stream(st):
+                A = sap.BandedMatrix(torch.from_numpy(b).cuda())
+                g = sap.Solver(1, sap.Options(**opts))
+                for _ in range(150):
+                    g.setup(A)
+                assert np.array_equal(g.factors(), ref)
+        except Exception as e:   # (reported by the main thread)
+            errors.append(e)
+    threads = [threading.Thread(target=work, args=x) for x in zip(bands, one)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors, errors
