@@ -81,3 +81,124 @@ def test_blocks_that_grow_are_substituted(sap, oracle, n, k, d):
     norm = np.abs(band).sum(axis=1).max()
     assert np.isfinite(z).all()
     assert np.abs(res).max() <= 1e-10 * norm * np.abs(z).max()
+
+
+def host_apply(F, v):
+    """M^{-1} v of one partition in FP64 from its factor band (row c: column c,
+    entry (r, c) at k + r - c): L, D, U'."""
+    n, k = len(F), F.shape[1] // 2
+    x = v.astype(np.float64)
+    for c in range(n):
+        m = min(k, n - 1 - c)
+        x[c + 1:c + 1 + m] -= F[c, k + 1:k + 1 + m] * x[c]
+    x /= F[:, k]
+    for c in range(n - 1, -1, -1):
+        m = min(k, c)
+        x[c - m:c] -= F[c, k - m:k] * x[c]
+    return x
+
+
+def host_inverse_max(F, bs):
+    """Largest entry of the inverse of each unit-lower diagonal block of bs rows."""
+    k = F.shape[1] // 2
+    out = []
+    for c0 in range(0, len(F) - bs + 1, bs):
+        L = np.eye(bs)
+        for j in range(bs):
+            m = min(k, bs - 1 - j)
+            L[j + 1:j + 1 + m, j] = F[c0 + j, k + 1:k + 1 + m]
+        out.append(np.abs(np.linalg.inv(L)).max())
+    return np.array(out)
+
+
+@pytest.mark.parametrize("n,k,d", [(1200, 20, 0.1), (1203, 33, 0.1), (1500, 50, 0.1), (1600, 90, 0.05),
+                                   (1601, 150, 0.05), (1500, 300, 0.02)])
+@pytest.mark.parametrize("prec_double", [True, False])
+def test_substitution_against_the_factors(sap, oracle, n, k, d, prec_double):
+    """The substituting blocks in both precisions, against the same factors
+    applied in FP64 on the host: the sweeps' own error alone.  Substitution
+    keeps |L D U' z - v| within about 2 k eps of |L| |D| |U'| |z| (a sum of k
+    products a row in either solve); the blocks that are multiplied may add
+    what their inverses' entries allow, so 8 k eps."""
+    print(f"[sweeps] factors n={n} k={k} d={d} fp64={prec_double}", flush=True)
+    band = oracle.gen_banded(n, k, d, 740 + k)
+    v = oracle.gen_vector(n, 741)
+    g = sap.Solver(1, sap.Options(precondType=sap.Block, factMethod=sap.LU_only, safeFactorization=1,
+                                  precValueType=sap.PREC_DOUBLE if prec_double else sap.PREC_FLOAT))
+    g.setup(sap.BandedMatrix(dev(band)))
+    z = torch.empty(n, dtype=torch.float64, device="cuda")
+    g.precond_apply(dev(v), z)
+    z = z.cpu().numpy()
+    F = g.factors()
+    grown = host_inverse_max(F, 16 if prec_double else 32)
+    assert (grown > 16).sum() >= 2, grown          # the branch is reached
+    # w = L D U' z through the factors, row sums of |L| |D| |U'| |z| beside it
+    def times(F, x, ab=lambda t: t):
+        y = ab(x).copy()
+        for c in range(n):                         # U' (unit upper)
+            m = min(k, c)
+            y[c - m:c] += ab(F[c, k - m:k]) * ab(x)[c]
+        y = y * ab(F[:, k])
+        w = y.copy()
+        for c in range(n):                         # L (unit lower)
+            m = min(k, n - 1 - c)
+            w[c + 1:c + 1 + m] += ab(F[c, k + 1:k + 1 + m]) * y[c]
+        return w
+    vt = v if prec_double else v.astype(np.float32).astype(np.float64)
+    eps = 2.0 ** -53 if prec_double else 2.0 ** -24
+    res = np.abs(times(F, z) - vt).max()
+    bound = times(F, z, np.abs).max()
+    print(f"[sweeps] backward error {res / bound / eps:.1f} eps, blocks grown {int((grown > 16).sum())}", flush=True)
+    assert res <= 8 * k * eps * bound
+    # and the value itself: n eps by the four decades these factors amplify
+    ref = host_apply(F, vt)
+    assert np.isfinite(z).all() and np.linalg.norm(z - ref) <= 1e-2 * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("k", [70, 96, 200])
+@pytest.mark.parametrize("prec_double", [True, False])
+def test_substitution_in_the_spike_passes(sap, oracle, k, prec_double):
+    """LU and UL factors of every partition, full sweeps in halves and interface
+    sweeps (k >= 70: every pivot boosted) with blocks that grow: the same
+    operator as with the plain sweeps (no memory for the tables), to rounding
+    by the four decades or so that these factors amplify."""
+    import os
+    n, P, d = 8 * k + 37, 3, 0.03
+    print(f"[sweeps] spike k={k} fp64={prec_double}", flush=True)
+    band, v = oracle.gen_banded(n, k, d, 760 + k), oracle.gen_vector(n, 761)
+    opts = dict(precondType=sap.Spike, factMethod=sap.LU_UL, safeFactorization=1,
+                precValueType=sap.PREC_DOUBLE if prec_double else sap.PREC_FLOAT)
+    z = apply(sap, band, v, P, **opts)
+    os.environ["SAP_AMD_DEVICE_FREE"] = "4"
+    try:
+        plain = apply(sap, band, v, P, **opts)
+    finally:
+        del os.environ["SAP_AMD_DEVICE_FREE"]
+    d = np.linalg.norm(z - plain) / np.linalg.norm(plain)
+    print(f"[sweeps] staged against plain {d:.2e}", flush=True)
+    assert np.isfinite(z).all() and d <= (1e-8 if prec_double else 1e-2)
+
+
+def test_substitution_costs_little_more(sap):
+    """A band whose blocks mostly grow may not sweep several times slower than
+    one of the same size without growth (the chain of substitutions is 31 steps
+    of a register broadcast and a multiply-add)."""
+    def us(d):
+        n, k, P = 100000, 20, 16
+        g = sap.Solver(P, sap.Options(precondType=sap.Block, safeFactorization=1))
+        g.setup(sap.BandedMatrix.generate(n, k, d, 7))
+        v = torch.ones(n, dtype=torch.float64, device="cuda")
+        z = torch.empty_like(v)
+        best = 1e9
+        for _ in range(8):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            for _ in range(5):
+                g.precond_apply(v, z)
+            b.record()
+            torch.cuda.synchronize()
+            best = min(best, a.elapsed_time(b) / 5 * 1e3)
+        return best
+    grown, plain = us(0.1), us(1.2)
+    print(f"[sweeps] {grown:.0f} us with growth, {plain:.0f} without", flush=True)
+    assert grown <= 3 * plain
