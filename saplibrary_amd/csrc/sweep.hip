@@ -699,7 +699,7 @@ __device__ __forceinline__ void lower_sweep_lds(const BandView<T>& V, const T* _
                 // on): substitute, element vi in each lane.  (The row comes
                 // to registers first: with a read per step of the chain, a
                 // band of n = 100000, k = 20, 16 partitions whose blocks mostly
-                // grow took 628 us in FP32, 550 in FP64; 211 and 312 so, 121
+                // grow took 628 us in FP32, 550 in FP64; 225 and 330 so, 119
                 // and 217 where none grows.)
                 T l[BS], y = p;
                 CM::lds_row(S.a + base, vi, l);
@@ -934,8 +934,20 @@ __device__ __forceinline__ void lower_sweep_lds(const BandView<T>& V, const T* _
 // in T, zero in S.  One BS-lane group per block: lane j solves for column j
 // of T with the block's multipliers broadcast from LDS.  A block of whose
 // inverse an entry passes SW_GROWTH (or is no number) keeps its multipliers
-// instead, T(0, 0) = 0 telling the sweeps to substitute: multiplying with T
-// loses up to about that growth in accuracy against substitution.
+// instead, T(0, 0) = 0 telling the sweeps to substitute: the product with T has
+// no small residual in the block's own equations, which the following blocks
+// then amplify.  The limit is where the error of a whole application (against
+// the same factors in higher precision) is still that of substituting
+// everywhere: the ratio of the two, geometric mean of 240 bands each with n =
+// 800, k = 20, 50 and 90 (+- 0.04), by the band's dominance:
+//               FP32 0.04   0.07   0.1    FP64 0.04   0.07   0.1
+//   limit 4          1.00   1.00   0.87        0.97   1.04   0.96
+//         8          0.99   1.05   0.86        0.99   1.04   0.97
+//        16          1.06   1.21   0.99        1.14   1.21   1.14
+// The error is smaller than substitution's where nothing grows (0.6 in FP32
+// and 0.8 in FP64 from 0.3 on, at every limit), and T in twice the precision
+// changes nothing.  A lower limit costs time on growing bands only: 211 us at
+// 16, 225 at 8, 228 at 4 (dominance 0.1, n = 100000, k = 20, FP32).
 // Bound by bytes, 264 written a row and direction and the lines that hold the
 // diagonal blocks read: 0.62 ms at n = 1000000, k = 200 with both
 // factorizations (1.06 GB written, 1.6 GB read), 52 us at n = 200000, k = 50.
@@ -943,7 +955,7 @@ __device__ __forceinline__ void lower_sweep_lds(const BandView<T>& V, const T* _
 // (0.58 and 0.79 ms saved on each).
 // ---------------------------------------------------------------------------
 constexpr int TAB_THREADS = 256;
-constexpr double SW_GROWTH = 16.0;
+constexpr double SW_GROWTH = 8.0;
 
 template <class T>
 __global__ __launch_bounds__(TAB_THREADS) void sweep_tables_kernel(const T* __restrict__ B0, const T* __restrict__ B1,
