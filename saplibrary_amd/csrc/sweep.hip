@@ -1424,7 +1424,12 @@ size_t sweep_lds(int k)
 struct SweepCfg { int mode, nbuf; size_t lds; int threads, depth; };
 
 // tabs_ok: the factorization's T blocks exist; depth_req: at most so many
-// slots (0: as many as fit)
+// slots (0: as many as fit).  As many as fit also where there are more
+// workgroups than CUs (several columns, job tables): three wavefronts of 121
+// to 126 registers per SIMD leave no CU room for a second workgroup, whatever
+// its LDS.  One sweep of 16 partitions, 16 columns with at most four slots and
+// with all: 271 and 149 us at k = 50 (n = 200000, FP32), 152 and 152 at k = 80,
+// 188 and 151 at k = 20 (n = 100000, FP64), 171 and 175 at k = 150.
 template <class T>
 SweepCfg sweep_cfg(int k, bool tabs_ok, int depth_req = 0)
 {
@@ -1464,8 +1469,7 @@ void launch_sweep_interface(const T* B, const T* Bul, const SweepTabs<T>& tabs, 
                             T* g, T* scr0, T* scr1, hipStream_t st, const Rhs& rh)
 {
     if (pi.P < 2) return;
-    // several columns: the fewest staging buffers, so more workgroups fit on a CU
-    const SweepCfg c = sweep_cfg<T>(k, tabs.lu1 != nullptr, rh.nr > 1 ? 4 : rh.nbuf);
+    const SweepCfg c = sweep_cfg<T>(k, tabs.lu1 != nullptr, rh.nbuf);
     if (c.mode == 2) launch_sweep_interface_t<T, 2>(B, Bul, tabs, k, pi, v, g, scr0, scr1, c, rh, st);
     else launch_sweep_interface_t<T, 0>(B, Bul, tabs, k, pi, v, g, scr0, scr1, c, rh, st);
 }
@@ -1504,7 +1508,7 @@ template <class T>
 void launch_sweep_full(const T* B, const T* Bul, const SweepTabs<T>& tabs, int k, PartInfo pi, int last_is_ul,
                        const double* v, const T* corr, double* outd, T* outt, T* scr, hipStream_t st, const Rhs& rh)
 {
-    const SweepCfg c = sweep_cfg<T>(k, tabs.lu1 != nullptr, rh.nr > 1 ? 4 : rh.nbuf);
+    const SweepCfg c = sweep_cfg<T>(k, tabs.lu1 != nullptr, rh.nbuf);
     if (c.mode == 2) launch_sweep_full_t<T, 2>(B, Bul, tabs, k, pi, last_is_ul, v, corr, outd, outt, scr, c, rh, st);
     else launch_sweep_full_t<T, 0>(B, Bul, tabs, k, pi, last_is_ul, v, corr, outd, outt, scr, c, rh, st);
 }
@@ -1524,8 +1528,7 @@ bool sweep_jobs_append(std::vector<SweepJob>& jobs, size_t& lds, const T* B, con
                        PartInfo pi, T* scr, int64_t voff, int64_t ldv, int64_t ooff, int64_t ldo, int nr, int gate0,
                        int* mode_out)
 {
-    // many workgroups: the fewest staging buffers, so more fit on a CU
-    const SweepCfg c = sweep_cfg<T>(k, tabs.lu1 != nullptr, 4);
+    const SweepCfg c = sweep_cfg<T>(k, tabs.lu1 != nullptr);
     if (k == 0) return false;
     if (mode_out) *mode_out = c.mode;
     else if (c.mode != 2) return false;
@@ -1565,7 +1568,7 @@ template <class T>
 int sweep_range_job_append(std::vector<SweepJob>& jobs, size_t& lds, const T* B, const SweepTabs<T>& tabs, int k,
                            int64_t s0, int64_t len0, T* scr, int64_t n, int64_t ldv, int64_t ldo, int nr)
 {
-    const SweepCfg c = sweep_cfg<T>(k, tabs.lu1 != nullptr, 4);
+    const SweepCfg c = sweep_cfg<T>(k, tabs.lu1 != nullptr);
     lds = std::max(lds, c.lds);
     for (int r = 0; r < nr; ++r) {
         SweepJob J{};
