@@ -139,16 +139,13 @@ __global__ __launch_bounds__(256) void band_factor_kernel(T* __restrict__ B0, T*
 //      one column step behind (multipliers shared through LDS);
 //   3. the k x k trailing window in global memory (L2) receives the rank-32
 //      update -L_below * U_right on the matrix cores
-//      (v_mfma_f64_16x16x4f64), tiles held transposed so that their loads and stores run along columns,
-//      four tiles per wavefront in flight; -L_below comes from LDS or, for
-//      the widest FP64 bands, from the band itself.
+//      (v_mfma_f64_16x16x4f64), tiles held transposed so that their loads
+//      and stores run along columns, four tiles per wavefront in flight;
+//      -L_below comes from LDS or, for the widest bands, from the band
+//      itself.
 // Factors are written as L (unit), D, U' (divided), like the LDS variant.
 // ---------------------------------------------------------------------------
-template <class T>
-struct Mfma;
-
-template <>
-struct Mfma<double> {
+struct Mfma {
     static constexpr int TILE = 16, KSTEP = 4, NACC = 4;
     typedef double acc_t __attribute__((ext_vector_type(4)));
     __device__ static inline acc_t mma(double a, double b, acc_t c)
@@ -167,13 +164,12 @@ constexpr int MNB = 32;   // panel width of the MFMA factorization
 // lg: the -L_below operand is read from the band (written one step
 // earlier by the same workgroup) instead of being staged in LDS, which
 // leaves the LDS to the U block alone (the wide bands).
-template <class T>
 struct MfmaLds {
     int kp, ls_stride, us_stride;
     size_t ls_off, us_off, ld_off, prow_off, piv_off, bytes;
     __host__ __device__ MfmaLds(int k, bool lg = false)
     {
-        constexpr int TILE = 16;
+        constexpr int TILE = Mfma::TILE;
         kp = ((k + TILE - 1) / TILE) * TILE;
         ls_stride = MNB + 1;
         us_stride = kp + 4;
@@ -182,18 +178,19 @@ struct MfmaLds {
         ld_off = us_off + (size_t)MNB * us_stride;
         prow_off = ld_off + (size_t)2 * MNB;
         piv_off = prow_off + 2 * MNB;
-        bytes = (piv_off + MNB) * sizeof(T);
+        bytes = (piv_off + MNB) * sizeof(double);
     }
 };
 
 // NT threads, one panel row and one U-block column each, so k + 32 <= NT.
 // LG: -L_below read from the band in the trailing update (MfmaLds lg).
 constexpr int NT = 512;
-template <class T, bool LG>
-__global__ __launch_bounds__(NT) void band_factor_mfma_kernel(T* __restrict__ B0, T* __restrict__ B1, int k_all,
-                                                               const FactorJob* __restrict__ jobs)
+template <bool LG>
+__global__ __launch_bounds__(NT) void band_factor_mfma_kernel(double* __restrict__ B0, double* __restrict__ B1,
+                                                               int k_all, const FactorJob* __restrict__ jobs)
 {
-    using MF = Mfma<T>;
+    using T = double;
+    using MF = Mfma;
     constexpr int TILE = MF::TILE;
     const FactorJob job = jobs[blockIdx.x];
     const int k = job.kb > 0 ? job.kb : k_all;
@@ -207,7 +204,7 @@ __global__ __launch_bounds__(NT) void band_factor_mfma_kernel(T* __restrict__ B0
 
     extern __shared__ unsigned char smem_raw[];
     T* sm = reinterpret_cast<T*>(smem_raw);
-    const MfmaLds<T> lay(k, LG);
+    const MfmaLds lay(k, LG);
     T* Ls = sm + lay.ls_off;       // -L_below [kp][MNB+1]
     T* Us = sm + lay.us_off;       // U_right [MNB][kp+4]
     T* lcol = sm + lay.ld_off;     // multipliers of one panel column for rows < MNB, [2][MNB]
@@ -1186,12 +1183,12 @@ constexpr size_t LDS_LIMIT = 160 * 1024 - 1024;   // leave room for static LDS
 
 }  // namespace
 
-template <class T, bool LG>
-void launch_factor_mfma(T* B0, T* B1, int k, const FactorJob* jobs, int njobs, hipStream_t st)
+template <bool LG>
+void launch_factor_mfma(double* B0, double* B1, int k, const FactorJob* jobs, int njobs, hipStream_t st)
 {
-    const size_t lds = MfmaLds<T>(k, LG).bytes;
-    set_lds_limit((const void*)band_factor_mfma_kernel<T, LG>, lds);
-    hipLaunchKernelGGL((band_factor_mfma_kernel<T, LG>), dim3(njobs), dim3(NT), lds, st, B0, B1, k, jobs);
+    const size_t lds = MfmaLds(k, LG).bytes;
+    set_lds_limit((const void*)band_factor_mfma_kernel<LG>, lds);
+    hipLaunchKernelGGL((band_factor_mfma_kernel<LG>), dim3(njobs), dim3(NT), lds, st, B0, B1, k, jobs);
     SAP_LAUNCH_CHECK();
 }
 
@@ -1205,8 +1202,8 @@ int factor_mfma_variant(int k)
 {
     if (band_factor_window_fits<T>(k)) return 100;
     if constexpr (sizeof(T) == 8) {
-        if (k + MNB <= NT && MfmaLds<T>(k).bytes <= LDS_LIMIT) return 101;
-        if (k + MNB <= NT && MfmaLds<T>(k, true).bytes <= LDS_LIMIT) return 102;
+        if (k + MNB <= NT && MfmaLds(k).bytes <= LDS_LIMIT) return 101;
+        if (k + MNB <= NT && MfmaLds(k, true).bytes <= LDS_LIMIT) return 102;
     }
     return -1;
 }
@@ -1233,8 +1230,8 @@ void launch_band_factor(T* B0, T* B1, const T* Bin, int k, const FactorJob* d_jo
     if (launch_band_factor_window<T>(B0, B1, k, d_jobs, njobs, st)) return;
     if constexpr (sizeof(T) == 8) {
         const int mv = factor_mfma_variant<T>(k);
-        if (mv == 101) { launch_factor_mfma<T, false>(B0, B1, k, d_jobs, njobs, st); return; }
-        if (mv == 102) { launch_factor_mfma<T, true>(B0, B1, k, d_jobs, njobs, st); return; }
+        if (mv == 101) { launch_factor_mfma<false>(B0, B1, k, d_jobs, njobs, st); return; }
+        if (mv == 102) { launch_factor_mfma<true>(B0, B1, k, d_jobs, njobs, st); return; }
     }
     if (factor_lds_bytes<T>(k, 32) <= LDS_LIMIT)      launch_factor_nb<T, 32>(B0, B1, k, d_jobs, njobs, st);
     else if (factor_lds_bytes<T>(k, 16) <= LDS_LIMIT) launch_factor_nb<T, 16>(B0, B1, k, d_jobs, njobs, st);

@@ -441,7 +441,11 @@ void launch_factor_resident(T* B0, T* B1, const T* Bin, int k, const FactorJob* 
 }
 
 // Largest window (in 16-row tiles) kept in registers: FP32 up to k = 224,
-// FP64 (twice the registers and LDS per tile) up to k = 112.
+// FP64 (twice the registers and LDS per tile) up to k = 112.  The two widest
+// FP64 windows spill (7 registers at k = 81 .. 96, 78 at k = 97 .. 112: 32 and
+// 124 bytes of scratch a lane) and are still faster than the kernel with the
+// window in the L2: 4.7 against 5.6 ms and 5.6 against 6.6 (n = 100000, 8
+// partitions); the next does not fit.
 template <class T>
 constexpr int resident_max_kt() { return sizeof(T) == 4 ? 16 : 9; }
 

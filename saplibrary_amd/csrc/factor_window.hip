@@ -23,14 +23,16 @@ namespace {
 //   C.  the panel's factors go out, and the trailing tiles are read, updated on
 //       the matrix cores and written back, two per wavefront at a time while
 //       the next two are loading.
-// What bounds it, FP64 at k = 150, of 56k cycles a panel: B 26k (issue of the
-// broadcast multiply-adds, two wavefronts on a SIMD), C 23k (the matrix cores
-// need 13.2k of it), A 10k (latency of the L2).  The columns that enter next
-// are read ahead from HBM during B (A and C together 42k without).  A thread
-// per panel row with a barrier per column, as this was done before, took 13.4
-// ms for LU and UL (n = 250007, k = 150, 32 partitions, FP64); this takes 5.9.
-// FP32, n = 100000, 16 partitions: 13.1 -> 4.8 ms at k = 230, 25.9 -> 11.9 at
-// k = 480.
+// What bounds it, FP64 at k = 150, of 62k cycles a panel with a clock read
+// between the phases (57k without): A 14k (latency of the L2), B 23k (issue of
+// the broadcast multiply-adds, two wavefronts on a SIMD), C 25k (the matrix
+// cores need 13.2k of it).  The columns that enter next are read ahead from
+// HBM during B (without: 6.8 ms instead of 5.9).  29 registers spill in FP32
+// (128 for each of 16 wavefronts) and 28 in FP64 (256 for each of 8), 120 and
+// 116 bytes of scratch a lane.  A thread per panel row with a barrier per
+// column, as this was done before, took 13.4 ms for LU and UL (n = 250007, k =
+// 150, 32 partitions, FP64); this takes 5.9.  FP32, n = 100000, 16 partitions:
+// 13.1 -> 4.8 ms at k = 230, 25.9 -> 11.9 at k = 480.
 // ---------------------------------------------------------------------------
 template <class T>
 struct WinGeom {

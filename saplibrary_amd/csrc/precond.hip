@@ -764,8 +764,8 @@ void Precond<T>::var_spikes()
         const int nc = std::min(chunk, ncol - c0);
         launch_var_rhs<T>(pi, k, sp_.get(), voffB(), voffC(), vperm_r_.get(), vperm_l_.get(), vwidth_.get(),
                           vcols_.get() + c0, nc, stride, V.get(), stream);
-        std::vector<SweepJob> by_mode[3];
-        size_t lds[3] = {0, 0, 0};
+        std::vector<SweepJob> by_mode[2];   // plain, staged
+        size_t lds[2] = {0, 0};
         for (int j = 0; j < nc; ++j) {
             const VarSpikeCol& c = vcols_h_[c0 + j];
             const int p = c.i + c.side;
@@ -776,21 +776,21 @@ void Precond<T>::var_spikes()
             const int mode = sweep_range_job_append<T>(one, l, Bv_.get() + vboff_[p], range_tabs(s, p), vks_[p], 0, len,
                                                        scr.get() + (int64_t)j * stride, len, 0, 0, 1);
             one[0].voff = one[0].ooff = (int64_t)j * stride;
-            by_mode[mode].push_back(one[0]);
-            lds[mode] = std::max(lds[mode], l);
+            by_mode[mode / 2].push_back(one[0]);
+            lds[mode / 2] = std::max(lds[mode / 2], l);
         }
         std::vector<SweepJob> jobs;
-        size_t start[3];
-        for (int m = 0; m < 3; ++m) {
+        size_t start[2];
+        for (int m = 0; m < 2; ++m) {
             start[m] = jobs.size();
             jobs.insert(jobs.end(), by_mode[m].begin(), by_mode[m].end());
         }
         SAP_HIP_CHECK(hipMemcpyAsync(jd.get(), jobs.data(), jobs.size() * sizeof(SweepJob), hipMemcpyHostToDevice,
                                      stream));
-        for (int m = 2; m >= 0; --m)
+        for (int m = 1; m >= 0; --m)
             if (!by_mode[m].empty())
                 launch_sweep_full_jobs<T>(jd.get() + start[m], (int)by_mode[m].size(), lds[m], V.get(), Z.get(),
-                                          nullptr, stream, m);
+                                          nullptr, stream, 2 * m);
         launch_var_tips<T>(pi, k, sp_.get(), vperm_r_.get(), vperm_l_.get(), vwidth_.get(), vcols_.get() + c0, nc,
                            stride, Z.get(), WV_.get(), stream);
         SAP_HIP_CHECK(hipStreamSynchronize(stream));   // the job table is rewritten, the buffers released
@@ -913,8 +913,8 @@ typename Precond<T>::VJobs& Precond<T>::var_jobs(int nr, int64_t ldv, int64_t ld
     if (key.nr == J.key.nr && key.ldv == J.key.ldv && key.ldz == J.key.ldz && key.scr == J.key.scr && J.n > 0)
         return J;
     const PartInfo pi{n, P};
-    // the jobs grouped by sweep variant (one launch each)
-    std::vector<SweepJob> by_mode[3];
+    // the jobs grouped by sweep variant, plain and staged (one launch each)
+    std::vector<SweepJob> by_mode[2];
     for (int p = 0; p < P; ++p) {
         int64_t s, len;
         pi.bounds(p, s, len);
@@ -925,11 +925,12 @@ typename Precond<T>::VJobs& Precond<T>::var_jobs(int nr, int64_t ldv, int64_t ld
         if (!sweep_jobs_append<T>(one, lds, Bp, range_tabs(s, p), vks_[p], PartInfo{len, 1}, scr + nr * s, s, ldv, s,
                                   ldz, nr, 0, &mode))
             throw Error(SAP_ERR_HIP, "variable-bandwidth sweep job table");
-        by_mode[mode].insert(by_mode[mode].end(), one.begin(), one.end());
-        J.lds[mode] = std::max(J.lds[mode], lds);
+        std::vector<SweepJob>& list = by_mode[mode / 2];
+        list.insert(list.end(), one.begin(), one.end());
+        J.lds[mode / 2] = std::max(J.lds[mode / 2], lds);
     }
     std::vector<SweepJob> jobs;
-    for (int m = 0; m < 3; ++m) {
+    for (int m = 0; m < 2; ++m) {
         J.start[m] = jobs.size();
         J.count[m] = by_mode[m].size();
         jobs.insert(jobs.end(), by_mode[m].begin(), by_mode[m].end());
@@ -947,9 +948,9 @@ template <class T>
 void Precond<T>::var_sweeps(const double* V, int64_t ldv, double* Z, int64_t ldz, int nr, const int* gate, T* scr)
 {
     const VJobs& J = var_jobs(nr, ldv, ldz, scr);
-    for (int m = 2; m >= 0; --m)
+    for (int m = 1; m >= 0; --m)
         if (J.count[m])
-            launch_sweep_full_jobs<T>(J.d.get() + J.start[m], (int)J.count[m], J.lds[m], V, Z, gate, stream, m);
+            launch_sweep_full_jobs<T>(J.d.get() + J.start[m], (int)J.count[m], J.lds[m], V, Z, gate, stream, 2 * m);
 }
 
 // getSRev's variable-bandwidth branch (sap/precond.h:1457-1470, then the
@@ -1171,7 +1172,6 @@ int Precond<T>::factor_band_steps()
     const bool check_pivots = !cfg.safeFactorization && !(boost && boost_last);
 
     begin_tables(P, k, lu_ul() && spike_active());
-    const size_t kk = (size_t)k * k;
     if (!spike_active()) {
         std::vector<FactorJob> jobs;
         for (int p = 0; p < P; ++p) {

@@ -297,7 +297,7 @@ private:
     struct VJobs {
         DevBuf<SweepJob> d;
         size_t n = 0;                       // jobs in d (0: not built)
-        size_t start[3] = {0, 0, 0}, count[3] = {0, 0, 0}, lds[3] = {0, 0, 0};   // per sweep variant
+        size_t start[2] = {0, 0}, count[2] = {0, 0}, lds[2] = {0, 0};   // plain, staged sweeps
         VJobKey key{0, 0, 0, nullptr};
     } vjobs_[2];
     VJobs& var_jobs(int nr, int64_t ldv, int64_t ldz, T* scr);

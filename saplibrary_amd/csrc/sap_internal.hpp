@@ -373,13 +373,11 @@ int sweep_max_nbuf(int k);
 // V and Z given at launch; gate[job.gate] switches a column off.
 struct SweepJob {
     const void* B;        // the system's factor band (null: a padding job)
-    const void* Bul;      // its UL band (last partition under LU_UL)
     const void *t1, *t2;  // its sweep tables (SweepTabs)
-    const void* corr;     // reduced-system corrections of this column, or null
     void* scr;            // n-element work vector of this column
     int64_t voff, ooff;
     int64_t n;
-    int P, k, part, gate, last_is_ul, ring_mask, nbuf, pad_;
+    int P, k, part, gate, ring_mask, nbuf;
     int64_t s0, len0;     // len0 > 0: band rows [s0, s0 + len0) instead of partition `part`
 };
 // Appends nr jobs (column r: input V + r*ldv, output Z + r*ldo, scratch

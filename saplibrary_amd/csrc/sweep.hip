@@ -1275,8 +1275,7 @@ __global__ __launch_bounds__(MODE == 2 ? SW_THREADS : 256) void sweep_full_jobs_
     if (gate && !gate[J.gate]) return;
     const PartInfo pi{J.n, J.P};
     const SweepTabs<T> tabs{(const T*)J.t1, (const T*)J.t2, (const T*)J.t1, (const T*)J.t2};
-    sweep_full_body<T, MODE>((const T*)J.B, (const T*)J.Bul, tabs, J.k, pi, J.last_is_ul, J.part, V + J.voff,
-                          (const T*)J.corr, Z + J.ooff, nullptr, (T*)J.scr, J.ring_mask, J.nbuf, pend, xblk, xblk2,
+    sweep_full_body<T, MODE>((const T*)J.B, (const T*)J.B, tabs, J.k, pi, 0, J.part, V + J.voff, nullptr, Z + J.ooff, nullptr, (T*)J.scr, J.ring_mask, J.nbuf, pend, xblk, xblk2,
                           -1, J.s0, J.len0);
 }
 
@@ -1543,10 +1542,8 @@ bool sweep_jobs_append(std::vector<SweepJob>& jobs, size_t& lds, const T* B, con
         SweepJob J{};
         if (part < pi.P) {
             J.B = B;
-            J.Bul = B;
             J.t1 = tabs.lu1;
             J.t2 = tabs.lu2;
-            J.corr = nullptr;
             J.scr = scr + (int64_t)r * pi.n;
             J.voff = voff + r * ldv;
             J.ooff = ooff + r * ldo;
@@ -1555,7 +1552,6 @@ bool sweep_jobs_append(std::vector<SweepJob>& jobs, size_t& lds, const T* B, con
             J.k = k;
             J.part = part;
             J.gate = gate0 + r;
-            J.last_is_ul = 0;
             J.ring_mask = ring_size(k) - 1;
             J.nbuf = c.nbuf;
         }
@@ -1573,10 +1569,8 @@ int sweep_range_job_append(std::vector<SweepJob>& jobs, size_t& lds, const T* B,
     for (int r = 0; r < nr; ++r) {
         SweepJob J{};
         J.B = B;
-        J.Bul = B;
         J.t1 = tabs.lu1;
         J.t2 = tabs.lu2;
-        J.corr = nullptr;
         J.scr = scr + (int64_t)r * n;
         J.voff = r * ldv;
         J.ooff = r * ldo;
@@ -1585,7 +1579,6 @@ int sweep_range_job_append(std::vector<SweepJob>& jobs, size_t& lds, const T* B,
         J.k = k;
         J.part = 0;
         J.gate = r;
-        J.last_is_ul = 0;
         J.ring_mask = ring_size(k) - 1;
         J.nbuf = c.nbuf;
         J.s0 = s0;
